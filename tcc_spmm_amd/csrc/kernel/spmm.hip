@@ -44,9 +44,9 @@
 // runs four waves per SIMD (128 registers each, accumulators included), F256 two (248 registers).
 //
 // Split SWs (reference src/kernel/spmm_kernel.cuh:228-282): a split task stores its row groups of
-// `task.mask` as 8-row partial tiles [tile][8][F]; lane 0 then takes, per slice, an agent-scope
-// acq_rel wrapping ticket on counters[sw * (F/128) + slice] with limit chunks - 1, so the counter
-// returns to zero by itself; the task whose ticket is chunks - 1 merges all partial tiles of the SW's
+// `task.mask` as 8-row partial tiles [tile][8][F]; lane 0 then releases them at agent scope and takes,
+// per slice, a wrapping ticket on counters[sw * (F/128) + slice] with limit chunks - 1, so the counter
+// returns to zero by itself; the task whose ticket is chunks - 1 acquires and merges all partial tiles of the SW's
 // slice in partialIds order starting from 0.0f and writes Y. No float atomics, no spin-waits.
 #include "spmm.h"
 #include "hip_support.h"
@@ -1107,16 +1107,22 @@ __device__ __forceinline__ void runTask(const KernelArgs& a, unsigned taskIndex)
     }
     if (!split) return;
 
-    // Completion tickets, one per slice: the acq_rel RMW at agent scope publishes this task's
-    // partial tiles and, for the last arriver, makes every other task's tiles visible (the XCD L2s
-    // are not coherent with each other, so the release writes back and the acquire invalidates).
+    // Completion tickets, one per slice: the release fence at agent scope publishes this task's
+    // partial tiles before its tickets, and the acquire fence of a last arriver makes every other
+    // task's tiles visible (the XCD L2s are not coherent with each other, so the release writes back
+    // and the acquire invalidates). Both work on the whole L2 of the XCD and cost every wave that runs
+    // there, so there is one release for all slices, and an acquire only where tiles are read. With an
+    // acq_rel ticket per slice instead, every split task invalidated its L2 once per slice (F256,
+    // 1M rows with 64 hub rows, 7,200 split tasks: 2,435 -> 1,923 us; a 262K-row power-law graph:
+    // 441 -> 401 us; 2.45M rows: 5,125 -> 5,005 us; F128, one ticket per task: no change).
     waveSync();
     if (lane == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
 #pragma unroll
         for (unsigned k = 0; k < S; ++k) {
             unsigned* counter = a.counters + std::size_t(sw) * S + k;
             const unsigned ticket =
-                __builtin_amdgcn_atomic_inc32(counter, task.chunks - 1, __ATOMIC_ACQ_REL, "agent");
+                __builtin_amdgcn_atomic_inc32(counter, task.chunks - 1, __ATOMIC_RELAXED, "agent");
             lastFlag[k] = ticket == task.chunks - 1;
         }
     }

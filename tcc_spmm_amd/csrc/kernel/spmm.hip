@@ -1,16 +1,16 @@
 // Fused INT8-dequantization SpMM for MI355X (gfx950, wave64): Y = A x tf32(dequant(X)).
 //
 // Work decomposition
-//   One workgroup per task (one Sw32Task: <= 384 panels of one 32-row SW), normally one wavefront;
-//   each XCD walks a contiguous range of the task list (xcdTask), balanced by panels when skewed,
+//   One workgroup per task (one Sw32Task: <= 384 panels of one 32-row SW), one wavefront on large
+//   plans; each XCD walks a contiguous range of the task list (xcdTask), balanced by panels when skewed,
 //   the range's last 512 tasks longest size class first (tailTask).
 //   The wave walks the task's panels once, in order, and accumulates all 32 rows x F features of
 //   the SW: four v_mfma_f32_32x32x8_f16 per panel and 128-feature slice (one per 32-feature block;
 //   M = features, N = the 32 rows, K = the panel's 8 slots) into 4 x 16 FP32 accumulators per
 //   slice. F256 runs both slices in the same wave, so the A side of a panel is loaded and built
 //   once, and takes its panels in pairs: four v_mfma_f32_32x32x16_f16 per pair and slice, K = the
-//   pair's 16 slots. Plans with few tasks for the chip take two waves per task instead, each walking half the
-//   panels, with the second wave's accumulators added by the first (runTask).
+//   pair's 16 slots. Plans with few tasks for the chip take two, four or eight waves per task instead
+//   (taskWaves), each walking its share of the panels; the write-back adds their accumulators (writeTask).
 //
 // Operands of one panel
 //   A (features x slots): the 8 slot rows of the X slice are gathered with one dwordx4 load per
@@ -44,9 +44,9 @@
 // runs four waves per SIMD (128 registers each, accumulators included), F256 two (248 registers).
 //
 // Split SWs (reference src/kernel/spmm_kernel.cuh:228-282): a split task stores its row groups of
-// `task.mask` as 8-row partial tiles [tile][8][F]; lane 0 then releases them at agent scope and takes,
-// per slice, a wrapping ticket on counters[sw * (F/128) + slice] with limit chunks - 1, so the counter
-// returns to zero by itself; the task whose ticket is chunks - 1 acquires and merges all partial tiles of the SW's
+// `task.mask` as 8-row partial tiles [tile][8][F]; lane 0 then takes, per slice, an agent-scope
+// acq_rel wrapping ticket on counters[sw * (F/128) + slice] with limit chunks - 1, so the counter
+// returns to zero by itself; the task whose ticket is chunks - 1 merges all partial tiles of the SW's
 // slice in partialIds order starting from 0.0f and writes Y. No float atomics, no spin-waits.
 #include "spmm.h"
 #include "hip_support.h"
@@ -63,6 +63,7 @@
 #include <stdexcept>
 #include <string>
 #include <type_traits>
+#include <utility>
 
 // A 4-byte load from a structured buffer (address = base + index x stride + offsets, range-checked
 // by index): the LLVM intrinsic behind the raw-buffer builtins, declared by its name since clang
@@ -105,6 +106,7 @@ struct KernelArgs {
     float* partials;
     unsigned* counters;
     unsigned rows, cols;
+    unsigned resident; // the whole grid runs at once, with slots to spare (launch)
     unsigned vec4; // y and partials are 16-byte aligned: stores and merge loads of 16 bytes
 #ifdef TCC_SPMM_TIMELINE
     unsigned long long* stamps; // measurement build only: [taskCount][4], see TaskClock
@@ -165,36 +167,48 @@ template <>
 struct Loader<kBuffer> {
     static constexpr bool kWide = false;
     __amdgpu_buffer_rsrc_t ids, meta, scales, x, vals;
-    unsigned first;     // task.begin: panel offsets are relative to it
-    unsigned vbase;     // value base of the task's first slot, the smallest of the task
+    const float* values; // of the whole matrix
+    unsigned first;     // the wave's first panel: panel offsets are relative to it
+    unsigned vbase;     // value base of the wave's first slot, the smallest of the wave
     unsigned xShift;    // log2(features)
 
     __device__ Loader(const KernelArgs& a, unsigned begin, unsigned end, unsigned features)
-        : first(begin), xShift(features == 256 ? 8u : 7u) {
+        : values(a.m.values), first(begin), vbase(0), xShift(features == 256 ? 8u : 7u) {
         const std::size_t slot0 = std::size_t(begin) * 8;
-        // Value bases grow in slot order (reference src/format/sw32.cpp:131-138) and every panel
-        // starts with a real slot, so the first slot of the task has the smallest base.
-        vbase = begin < end ? unsigned(a.m.sourceMetadata[slot0] >> 32) : 0u;
+        // Sized to the panels [begin, end): a pair's second panel past the end reads 0 (source 0, no
+        // entries) without a clamp.
         ids = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned*>(a.m.sourceIds + slot0), 0,
-                                                0x7FFFFFF0, 0x00020000);
+                                                (end - begin) * 32u, 0x00020000);
         meta = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<std::uint64_t*>(a.m.sourceMetadata + slot0), 0, 0x7FFFFFF0, 0x00020000);
-        vals = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.m.values + vbase), 4,
-                                                 0x7FFFFFF0, 0x00020000);
+            const_cast<std::uint64_t*>(a.m.sourceMetadata + slot0), 0, (end - begin) * 64u, 0x00020000);
+        rebase(0);
         scales = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.scales), 4, a.cols, 0x00020000);
         x = __builtin_amdgcn_make_buffer_rsrc(const_cast<std::int8_t*>(a.packedX), 0,
                                               a.cols << xShift, 0x00020000);
     }
-    __device__ Meta meta8(unsigned panel, unsigned lane) const {
-        const int off = int((panel - first) * 32u);
+    // Addresses the values from value base `base` on.
+    __device__ void rebase(unsigned base) {
+        vbase = base;
+        vals = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(values + base), 4, 0x7FFFFFF0,
+                                                 0x00020000);
+    }
+    // Before the first value loads; `m` is the metadata of the wave's first panel. Value bases grow in
+    // slot order (reference src/format/sw32.cpp:131-138) and every panel starts with a real slot, so
+    // that panel's first slot (lane 0) has the smallest base. It comes with the metadata the walk loads
+    // anyway; a load of its own would be one more dependent load before the first panel.
+    __device__ void startTask(const Meta& m) { rebase(__builtin_amdgcn_readfirstlane(m.base)); }
+    // Panel `panel`, clamped to `last` (the offset is scalar).
+    __device__ Meta meta8(unsigned panel, unsigned last, unsigned lane) const {
+        const int off = int((min(panel, last) - first) * 32u);
         const auto md = __builtin_amdgcn_raw_buffer_load_b64(meta, (lane & 7) * 8, 2 * off, kNt);
         return {__builtin_amdgcn_raw_buffer_load_b32(ids, (lane & 7) * 4, off, kNt), md[0], md[1]};
     }
-    // Panels q and q + 1, each clamped to `last`: one load per array for both.
+    // Panels q (clamped to `last`) and q + 1: one load per array for both. The range check counts the
+    // scalar offset.
     __device__ MetaPair meta2(unsigned q, unsigned last, unsigned lane) const {
-        const unsigned off = (min(q + ((lane >> 3) & 1u), last) - first) * 32u + (lane & 7) * 4;
-        const auto md = __builtin_amdgcn_raw_buffer_load_b64(meta, 2 * off, 0, kNt);
-        return {__builtin_amdgcn_raw_buffer_load_b32(ids, off, 0, kNt), md[0], md[1]};
+        const int off = int((min(q, last) - first) * 32u);
+        const auto md = __builtin_amdgcn_raw_buffer_load_b64(meta, (lane & 15) * 8, 2 * off, kNt);
+        return {__builtin_amdgcn_raw_buffer_load_b32(ids, (lane & 15) * 4, off, kNt), md[0], md[1]};
     }
     // scales and values are structured buffers of 4-byte records, addressed by index (no shift) and
     // range-checked by index: an index past the records reads 0.
@@ -216,26 +230,35 @@ struct Loader {
     static_assert(Addr == kGlobal || Addr == kGlobalU16, "64-bit addressing modes");
     static constexpr bool kWide = true;
     const KernelArgs* a;
-    unsigned features;
+    // Uniform bases, so that a load takes a scalar base and a 32-bit lane offset.
+    const unsigned* ids;       // of the wave's first panel
+    const std::uint64_t* meta;
+    const float* vals;         // from value base vbase on
+    unsigned first, vbase, features; // first, vbase: as in the buffer loader
 
-    __device__ Loader(const KernelArgs& args, unsigned, unsigned, unsigned f)
-        : a(&args), features(f) {}
-    __device__ Meta meta8(unsigned panel, unsigned lane) const {
-        const std::size_t first = std::size_t(panel) * 8;
-        const std::uint64_t md =
-            __builtin_nontemporal_load(a->m.sourceMetadata + first + (lane & 7));
-        return {__builtin_nontemporal_load(a->m.sourceIds + first + (lane & 7)), unsigned(md),
-                unsigned(md >> 32)};
+    __device__ Loader(const KernelArgs& args, unsigned begin, unsigned, unsigned f)
+        : a(&args), ids(args.m.sourceIds + std::size_t(begin) * 8),
+          meta(args.m.sourceMetadata + std::size_t(begin) * 8), vals(args.m.values), first(begin),
+          vbase(0), features(f) {}
+    __device__ void startTask(const Meta& m) {
+        vbase = __builtin_amdgcn_readfirstlane(m.base);
+        vals = a->m.values + vbase;
+    }
+    // Panel `panel`, and panels q and q + 1, clamped to `last`.
+    __device__ Meta meta8(unsigned panel, unsigned last, unsigned lane) const {
+        const unsigned s = (min(panel, last) - first) * 8 + (lane & 7);
+        const std::uint64_t md = __builtin_nontemporal_load(meta + s);
+        return {__builtin_nontemporal_load(ids + s), unsigned(md), unsigned(md >> 32)};
     }
     __device__ MetaPair meta2(unsigned q, unsigned last, unsigned lane) const {
-        const std::size_t s = std::size_t(min(q + ((lane >> 3) & 1u), last)) * 8 + (lane & 7);
-        const std::uint64_t md = __builtin_nontemporal_load(a->m.sourceMetadata + s);
-        return {__builtin_nontemporal_load(a->m.sourceIds + s), unsigned(md), unsigned(md >> 32)};
+        const unsigned s = (min(q + ((lane >> 3) & 1u), last) - first) * 8 + (lane & 7);
+        const std::uint64_t md = __builtin_nontemporal_load(meta + s);
+        return {__builtin_nontemporal_load(ids + s), unsigned(md), unsigned(md >> 32)};
     }
     __device__ float scale(unsigned src) const { return a->scales[min(src, a->cols - 1)]; }
-    // values[idx] (absent entries are masked by Stage::bits).
-    __device__ float value(unsigned idx, bool) const {
-        return __builtin_nontemporal_load(a->m.values + idx);
+    // values[idx] when `present`, else some value (absent entries are masked by Stage::bits).
+    __device__ float value(unsigned idx, bool present) const {
+        return __builtin_nontemporal_load(vals + (present ? idx - vbase : 0u));
     }
     __device__ u32x4 tile(unsigned src, unsigned lane, unsigned k) const {
         const std::int8_t* p =
@@ -252,40 +275,40 @@ struct Loader {
     }
 };
 
-// Panel kinds: G = 0..3, a bucket exclusive to row group G (known at compile time); kShared, a
-// shared bucket whose row groups `groups` are known at run time.
-constexpr unsigned kShared = 4;
-
+// Panel kinds: exclusive (a bucket of one row group, known per panel from the bucket bounds) and
+// shared (a bucket of several row groups, `groups`).
 struct Stage {     // one panel, ready to compute
     float scale;   // lane L: scale of slot L & 7
-    float v[4];    // lane L: raw A value of (slot L & 7, row 8g + (L >> 3)); v[0] for kind G < 4
+    float v[4];    // lane L: raw A value of (slot L & 7, row 8g + (L >> 3)); v[0] when exclusive
     unsigned bits; // bit g: that entry is present (wide loader only; narrow reads 0 instead)
     u32x4 x[2];    // 16-byte tile L & 7 of the X row of slot L >> 3, per slice of the wave
 };
 
-// Stage 2 of one panel of kind G (row groups `groups` when G == kShared), with the X tiles of the
+// Where an exclusive panel's entries are: lane L's row bit in the slot masks, 1 << (8g + (L >> 3))
+// for the panel's row group g, and the bits below it.
+struct RowBit {
+    unsigned at, below;
+};
+
+// Stage 2 of one panel (exclusive: `rowBit`; shared: row groups `groups`), with the X tiles of the
 // wave's S slices; the scale too unless the caller loads it (LoadScale false).
-template <unsigned G, unsigned S, class Ld, bool LoadScale = true>
-__device__ __forceinline__ void loadStage(const Ld& ld, const Meta& m, unsigned groups,
-                                          unsigned lane, Stage& s) {
+template <bool Shared, unsigned S, class Ld, bool LoadScale = true>
+__device__ __forceinline__ void loadStage(const Ld& ld, const Meta& m, const RowBit& rowBit,
+                                          unsigned groups, unsigned lane, Stage& s) {
     // Padding slots (source UINT32_MAX, metadata 0) have an empty row mask; their scale and X tile
     // read 0 (narrow) or a clamped row (wide), multiplied by A entries that are all 0.
     if constexpr (LoadScale) s.scale = ld.scale(m.id);
     s.bits = 0;
-    constexpr unsigned kCount = G < 4 ? 1 : 4;
+    constexpr unsigned kCount = Shared ? 4 : 1;
 #pragma unroll
     for (unsigned j = 0; j < kCount; ++j) {
-        const unsigned g = G < 4 ? G : j;
-        const unsigned row = g * 8 + (lane >> 3);
-        const bool present = ((m.mask >> row) & 1u) && (G < 4 || ((groups >> g) & 1u));
+        const unsigned at = Shared ? 1u << (j * 8 + (lane >> 3)) : rowBit.at;
+        const unsigned below = Shared || Ld::kWide ? at - 1u : rowBit.below;
+        const bool present = (m.mask & at) != 0 && (!Shared || ((groups >> j) & 1u));
         // The k-th set row bit of a slot owns values[base + k].
-        const unsigned idx = m.base + __popc(m.mask & ((1u << row) - 1u));
-        if constexpr (Ld::kWide) {
-            s.v[j] = ld.value(present ? idx : m.base, true);
-            s.bits |= unsigned(present) << j;
-        } else {
-            s.v[j] = ld.value(idx, present);
-        }
+        const unsigned idx = m.base + __popc(m.mask & below);
+        s.v[j] = ld.value(idx, present);
+        if constexpr (Ld::kWide) s.bits |= unsigned(present) << j;
     }
     // Lane L gathers slot L >> 3's row, whose source lane L >> 3 holds: a cross-lane permute instead
     // of a second sourceIds load (one vector memory instruction fewer per panel, 2% at c3 F128).
@@ -344,10 +367,6 @@ __device__ __forceinline__ float stageTf32(const Stage& s, unsigned j) {
     return (Wide && !((s.bits >> j) & 1u)) ? 0.0f : roundTf32(s.v[j]); // tf32(0) = 0
 }
 
-// Per lane: slot k = lane & 7, row (lane >> 3) of each row group; its table index in row group g
-// is (8g + (lane >> 3)) * 8 + k = 64g + lane. Kind G < 4 writes only row group G (the others hold
-// 0 for the whole bucket). Returns whether every entry of the panel has an exact f16 a'
-// (wave-uniform); if not, the panel contributes nothing here.
 // m * 2^-kXShift for a scale s = m * 2^e (m in [0.5, 1)): the sign and mantissa bits of s under the
 // biased exponent 126 - kXShift. One v_and_or_b32 (as cheap as a v_frexp_mant); a VOP3 takes no
 // literal and one scalar operand on gfx950, so the caller keeps the mask 0x807FFFFF in a VGPR
@@ -371,7 +390,7 @@ struct LaneMh {
 // moved the result through a VGPR and compared it again.
 __device__ __forceinline__ std::uint64_t normalF16(_Float16 v) {
     std::uint64_t mask;
-    asm("v_cmp_class_f16_e64 %0, %1, %2" : "=s"(mask) : "v"(v), "v"(0x108u));
+    asm("v_cmp_class_f16_e64 %0, %1, %2" : "=s"(mask) : "v"(v), "s"(0x108u));
     return mask;
 }
 
@@ -412,13 +431,13 @@ __device__ __forceinline__ unsigned xTile(unsigned slot, unsigned block) {
     return (slot * kBlocks + block) * 8;
 }
 
-// Writes panel `s` of kind G to LDS area `area`. Per lane: slot lane & 7, row lane >> 3 of each
-// row group; kind G < 4 writes only row group G (the others hold 0 for the whole bucket). Returns
-// whether every entry of the panel has an exact f16 a' (wave-uniform); if not, its table is all
-// zero, so the panel contributes nothing here.
-template <bool Wide, unsigned G, unsigned S>
+// Writes panel `s` to LDS area `area`. Per lane: slot lane & 7, row lane >> 3 of each row group; an
+// exclusive panel writes only its own row group, whose table entry of this lane is `entry` (the
+// other groups' entries hold 0). Returns whether every entry of the panel has an exact f16 a'
+// (wave-uniform); if not, its table is all zero, so the panel contributes nothing here.
+template <bool Wide, bool Shared, unsigned S>
 __device__ __forceinline__ bool stagePanel(const Stage& s, unsigned lane, const Lds& lds, unsigned area,
-                                           unsigned keep) {
+                                           unsigned entry, unsigned keep) {
     // 2^(e + kShift) for the slot's scale s = m * 2^e (m in [0.5, 1)): its exponent bits alone are
     // 2^(e - 1). A zero or subnormal scale gives 0 and an infinite or NaN one inf, so that every
     // nonzero entry of such a slot fails the check below and the panel takes the FP32 path (the
@@ -426,7 +445,7 @@ __device__ __forceinline__ bool stagePanel(const Stage& s, unsigned lane, const 
     const float pow2 = __builtin_amdgcn_ldexpf(__uint_as_float(__float_as_uint(s.scale) & 0x7F800000u),
                                                kShift + 1);
     std::uint64_t inexact = 0; // lanes with an entry that has no exact f16 a'
-    constexpr unsigned kCount = G < 4 ? 1 : 4;
+    constexpr unsigned kCount = Shared ? 4 : 1;
     _Float16 ap[kCount];
 #pragma unroll
     for (unsigned j = 0; j < kCount; ++j) {
@@ -445,7 +464,7 @@ __device__ __forceinline__ bool stagePanel(const Stage& s, unsigned lane, const 
     const bool useF16 = inexact == 0;
 #pragma unroll
     for (unsigned j = 0; j < kCount; ++j)
-        lds.table16[tableEntry<S>(G < 4 ? G : j, lane, area)] =
+        lds.table16[Shared ? tableEntry<S>(j, lane, area) : entry] =
             useF16 ? ap[j] : static_cast<_Float16>(0.0f);
 #pragma unroll
     for (unsigned k = 0; k < S; ++k) lds.xtile[xTile<S>(lane >> 3, S * area + k) + (lane & 7)] = s.x[k];
@@ -537,10 +556,11 @@ __device__ __forceinline__ void crunch(const Lds& lds, f32x16 (&acc)[4 * S], Lan
 }
 
 // One panel alone: staged in area 0 and computed.
-template <bool Wide, unsigned G, unsigned S>
+template <bool Wide, bool Shared, unsigned S>
 __device__ __forceinline__ bool computePanelF16(const Stage& s, unsigned lane, const Lds& lds,
-                                                f32x16 (&acc)[4 * S], unsigned keep, LaneMh mh) {
-    const bool useF16 = stagePanel<Wide, G, S>(s, lane, lds, 0, keep);
+                                                f32x16 (&acc)[4 * S], unsigned entry, unsigned keep,
+                                                LaneMh mh) {
+    const bool useF16 = stagePanel<Wide, Shared, S>(s, lane, lds, 0, entry, keep);
     crunch<S, false>(lds, acc, mh);
     return useF16;
 }
@@ -623,9 +643,33 @@ __device__ __forceinline__ void flagRedo(TaskWalk& w, unsigned panel, bool redo)
     }
 }
 
-// The panels [lo, hi) of kind G, pipelined, two panels per iteration with the odd one after the
-// loop (a single exit keeps the accumulators in place). Panel indices past the end repeat the last
-// panel (harmless loads, never computed).
+// Ends of the exclusive buckets of row groups 0..2 (group 3's is the end of the walk).
+struct GroupBounds {
+    unsigned b0, b1, b2;
+    __device__ unsigned end(unsigned g) const {
+        return g == 0 ? b0 : g == 1 ? b1 : g == 2 ? b2 : 0xFFFFFFFFu;
+    }
+};
+
+// Row group of the exclusive panels of one task, walked in increasing panel order. Wave-uniform, in
+// scalar registers: a panel inside the current bucket costs one compare and an untaken branch.
+struct GroupCursor {
+    unsigned g, end;
+    __device__ void advance(const GroupBounds& b, unsigned p) {
+        while (p >= end) end = b.end(++g);
+    }
+};
+
+// The panels [lo, hi) of one kind, pipelined, two panels per iteration with the odd one after the
+// loop (a single exit keeps the accumulators in place). The loads run past the end of the walk: they
+// read the next bucket's panels, nothing or the last panel again (Loader), and are never computed.
+// `first` is panel lo's metadata, loaded by the caller if
+// lo is the task's first panel (beside the bucket bounds, one dependent load earlier).
+//
+// The four exclusive buckets are one walk: the loads run ahead across a bucket's end, and only the
+// row bit of the loads and the table entry of the writes change there (wave-uniform branches, taken
+// at most three times a task). One loop per bucket instead emptied the pipeline four times per task,
+// about 2 us of cold loads each.
 //
 // F128 (S == 1) loads the metadata, sourceIds and scales of two panels with one instruction each, one
 // iteration ahead, and hands each panel its slots by DPP row shifts: per panel that is one and
@@ -634,85 +678,115 @@ __device__ __forceinline__ void flagRedo(TaskWalk& w, unsigned panel, bool redo)
 // gathers in flight: stage data two panels ahead, metadata four (1.2% faster than one panel ahead;
 // three ahead gained 0.2% for 16 more registers), and computes its panels in pairs, K = 16 per MFMA
 // (c3: 5.92 -> 5.72 ms).
-template <unsigned G, unsigned S, class Ld>
-__device__ __forceinline__ void walkPanels(const Ld& ld, TaskWalk& w, unsigned lo,
-                                           unsigned hi, f32x16 (&acc)[4 * S]) {
+template <bool Shared, unsigned S, class Ld>
+__device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBounds& bounds,
+                                           unsigned lo, unsigned hi, Meta first,
+                                           f32x16 (&acc)[4 * S]) {
     if (lo >= hi) return;
+    constexpr unsigned kAreas = S == 1 ? 1 : 2;
     const unsigned n = hi - lo, lane = w.lane;
-    if constexpr (G < 4) {
-        // The other row groups' table rows (64 entries each per area) stay 0 for the whole bucket.
-#pragma unroll
-        for (unsigned g = 0; g < 4; ++g) {
-            if (g == G) continue;
-            if constexpr (S == 1)
-                w.lds.table16[64 * g + lane] = static_cast<_Float16>(0.0f);
-            else // both areas: 128 entries, two per lane
-                reinterpret_cast<f16x2*>(w.lds.table16)[64 * g + lane] = f16x2{0, 0};
-        }
-    }
-    BucketCursor cur{w.offsets, 5, w.offsets[6]};
-    auto groupsAt = [&](unsigned p) { return G < 4 ? (1u << G) : cur.groups(p); };
     const unsigned last = hi - 1;
     const unsigned pairs = n / 2;
+    // The loads' side of a bucket change: to be called before the loads of panel p, for increasing p.
+    // Returns a shared panel's row groups.
+    BucketCursor bucket{w.offsets, 5, Shared ? w.offsets[6] : 0u};
+    GroupCursor loads{0, bounds.b0};
+    loads.advance(bounds, lo);
+    const unsigned bit0 = 1u << (lane >> 3);
+    RowBit rowBit{bit0 << (8 * loads.g), (bit0 << (8 * loads.g)) - 1u};
+    auto enter = [&](unsigned p) __attribute__((always_inline)) {
+        if constexpr (Shared) return bucket.groups(min(p, last));
+        if (__builtin_expect(p >= loads.end, 0)) {
+            loads.advance(bounds, p);
+            rowBit.at = bit0 << (8 * loads.g);
+            rowBit.below = rowBit.at - 1u;
+        }
+        return 0u;
+    };
+    // The table's side: an area's table holds one row group at a time, the other groups' entries 0.
+    GroupCursor staged[kAreas];
+    unsigned entry[kAreas];
+#pragma unroll
+    for (unsigned a = 0; a < kAreas; ++a) {
+        staged[a] = loads;
+        entry[a] = tableEntry<S>(loads.g, lane, a);
+    }
+    if constexpr (!Shared) {
+#pragma unroll
+        for (unsigned i = 0; i < 2 * kAreas; ++i)
+            reinterpret_cast<f16x2*>(w.lds.table16)[64 * i + lane] = f16x2{0, 0};
+    }
+    auto enterTable = [&](unsigned p, unsigned a) __attribute__((always_inline)) {
+        if constexpr (!Shared) {
+            if (__builtin_expect(p >= staged[a].end, 0)) {
+                w.lds.table16[entry[a]] = static_cast<_Float16>(0.0f);
+                staged[a].advance(bounds, p);
+                entry[a] = tableEntry<S>(staged[a].g, lane, a);
+            }
+        }
+    };
+    // Panel p alone, in area 0.
+    auto computeOne = [&](const Stage& st, unsigned p) __attribute__((always_inline)) {
+        enterTable(p, 0);
+        flagRedo(w, p, !computePanelF16<Ld::kWide, Shared, S>(st, lane, w.lds, acc, entry[0], w.keep, w.mh));
+    };
     Stage sa, sb;
-    unsigned ga = groupsAt(lo), gb = 0;
-    loadStage<G, S>(ld, ld.meta8(lo, lane), ga, lane, sa);
+    if (lo != w.begin) first = ld.meta8(lo, lo, lane);
     if constexpr (S == 1) {
-        MetaPair pair = ld.meta2(min(lo + 1, last), last, lane); // panels lo + 1, lo + 2
+        MetaPair pair = ld.meta2(lo + 1, last, lane); // panels lo + 1, lo + 2
+        __builtin_amdgcn_sched_barrier(0);
+        if (lo == w.begin) ld.startTask(first);
+        loadStage<Shared, S>(ld, first, rowBit, enter(lo), lane, sa);
         // Each panel's row shifts run half an iteration before its loads need them.
         Meta mFirst = pairPanel<0>(pair);
 #pragma unroll 1
         for (unsigned k = 0; k < pairs; ++k) {
             // Computes panels lo + 2k (in sa) and lo + 2k + 1; loads the pair after next.
-            const MetaPair next = ld.meta2(min(lo + 2 * k + 3, last), last, lane);
+            const unsigned gb = enter(lo + 2 * k + 1);
+            const MetaPair next = ld.meta2(lo + 2 * k + 3, last, lane);
             const float sc = ld.scale(pair.id); // both panels' scales, laid out as `pair`
-            gb = groupsAt(min(lo + 2 * k + 1, last));
-            loadStage<G, S, Ld, false>(ld, mFirst, gb, lane, sb);
+            loadStage<Shared, S, Ld, false>(ld, mFirst, rowBit, gb, lane, sb);
             const Meta mSecond = pairPanel<1>(pair);
             // Issue this half's loads before any use of the previous half's: the vmcnt counter
             // is in order, so computing first would wait for loads issued only half an
             // iteration ago.
             __builtin_amdgcn_sched_barrier(0);
-            flagRedo(w, lo + 2 * k, !computePanelF16<Ld::kWide, G, S>(sa, lane, w.lds, acc, w.keep, w.mh));
-            ga = groupsAt(min(lo + 2 * k + 2, last));
-            loadStage<G, S, Ld, false>(ld, mSecond, ga, lane, sa);
+            computeOne(sa, lo + 2 * k);
+            const unsigned ga = enter(lo + 2 * k + 2);
+            loadStage<Shared, S, Ld, false>(ld, mSecond, rowBit, ga, lane, sa);
             __builtin_amdgcn_sched_barrier(0);
             sb.scale = __uint_as_float(pairHalf<0>(__float_as_uint(sc)));
-            flagRedo(w, lo + 2 * k + 1, !computePanelF16<Ld::kWide, G, S>(sb, lane, w.lds, acc, w.keep, w.mh));
+            computeOne(sb, lo + 2 * k + 1);
             sa.scale = __uint_as_float(pairHalf<1>(__float_as_uint(sc)));
             pair = next;
             mFirst = pairPanel<0>(pair);
         }
-        if (n & 1) flagRedo(w, last, !computePanelF16<Ld::kWide, G, S>(sa, lane, w.lds, acc, w.keep, w.mh));
+        if (n & 1) computeOne(sa, last);
     } else {
         // F256: stage data two panels ahead, metadata four. Three stage buffers rotate: at the step
-        // of panel i they hold panels i, i + 1 and (loaded there) i + 2. Loads past the last panel
-        // repeat it (harmless, never computed).
+        // of panel i they hold panels i, i + 1 and (loaded there) i + 2.
         Stage sc;
-        unsigned gc = 0;
-        const unsigned p1 = min(lo + 1, last), p2 = min(lo + 2, last), p3 = min(lo + 3, last);
-        gb = groupsAt(p1);
-        loadStage<G, S>(ld, ld.meta8(p1, lane), gb, lane, sb);
-        unsigned g1 = groupsAt(p2), g2 = groupsAt(p3);
+        const Meta second = ld.meta8(lo + 1, last, lane);
         // The steps expect m1's loads to be older than m2's (waits are counted in issue order).
-        Meta m1 = ld.meta8(p2, lane);
+        Meta m1 = ld.meta8(lo + 2, last, lane);
         __builtin_amdgcn_sched_barrier(0);
-        Meta m2 = ld.meta8(p3, lane);
-        unsigned p = p3;
+        Meta m2 = ld.meta8(lo + 3, last, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        if (lo == w.begin) ld.startTask(first);
+        loadStage<Shared, S>(ld, first, rowBit, enter(lo), lane, sa);
+        loadStage<Shared, S>(ld, second, rowBit, enter(lo + 1), lane, sb);
         // Step of panel `panel` (in `cur`): the loads of panel + 2 into `ahead`, then the panel staged
         // in area 0 (first of a pair) or staged in area 1 and the pair computed (second).
-        auto step = [&](auto second, Stage& cur, Stage& ahead, unsigned& gahead,
+        auto step = [&](auto second, Stage& cur, Stage& ahead,
                         unsigned panel) __attribute__((always_inline)) {
-            gahead = g1;
-            loadStage<G, S>(ld, m1, gahead, lane, ahead);
-            p = min(p + 1, last);
+            loadStage<Shared, S>(ld, m1, rowBit, enter(panel + 2), lane, ahead);
             m1 = m2;
-            g1 = g2;
-            g2 = groupsAt(p);
-            m2 = ld.meta8(p, lane);
+            m2 = ld.meta8(panel + 4, last, lane);
             __builtin_amdgcn_sched_barrier(0);
             constexpr bool kSecond = decltype(second)::value;
-            flagRedo(w, panel, !stagePanel<Ld::kWide, G, S>(cur, lane, w.lds, kSecond ? 1u : 0u, w.keep));
+            constexpr unsigned kArea = kSecond ? 1u : 0u;
+            enterTable(panel, kArea);
+            flagRedo(w, panel, !stagePanel<Ld::kWide, Shared, S>(cur, lane, w.lds, kArea, entry[kArea], w.keep));
             if constexpr (kSecond) crunch<S, true>(w.lds, acc, w.mh);
         };
         using First = std::integral_constant<bool, false>;
@@ -725,33 +799,31 @@ __device__ __forceinline__ void walkPanels(const Ld& ld, TaskWalk& w, unsigned l
         unsigned i = lo;
 #pragma unroll 1
         for (unsigned k = 0; k < sixes; ++k, i += 6) {
-            step(First{}, sa, sc, gc, i);
-            step(Second{}, sb, sa, ga, i + 1);
-            step(First{}, sc, sb, gb, i + 2);
-            step(Second{}, sa, sc, gc, i + 3);
-            step(First{}, sb, sa, ga, i + 4);
-            step(Second{}, sc, sb, gb, i + 5);
+            step(First{}, sa, sc, i);
+            step(Second{}, sb, sa, i + 1);
+            step(First{}, sc, sb, i + 2);
+            step(Second{}, sa, sc, i + 3);
+            step(First{}, sb, sa, i + 4);
+            step(Second{}, sc, sb, i + 5);
         }
         if (r >= 2) {
-            step(First{}, sa, sc, gc, i);
-            step(Second{}, sb, sa, ga, i + 1);
+            step(First{}, sa, sc, i);
+            step(Second{}, sb, sa, i + 1);
         }
         if (r >= 4) {
-            step(First{}, sc, sb, gb, i + 2);
-            step(Second{}, sa, sc, gc, i + 3);
+            step(First{}, sc, sb, i + 2);
+            step(Second{}, sa, sc, i + 3);
         }
-        if (r & 1) {
-            const Stage& odd = r == 1 ? sa : r == 3 ? sc : sb;
-            flagRedo(w, hi - 1, !computePanelF16<Ld::kWide, G, S>(odd, lane, w.lds, acc, w.keep, w.mh));
-        }
+        if (r & 1) computeOne(r == 1 ? sa : r == 3 ? sc : sb, hi - 1);
     }
 }
 
 template <unsigned S, class Ld>
-__device__ __forceinline__ void walkTask(const Ld& ld, const unsigned* offsets, unsigned begin,
+__device__ __forceinline__ void walkTask(Ld& ld, const unsigned* offsets, unsigned begin,
                                          unsigned end, unsigned lane, const Lds& lds,
                                          f32x16 (&acc)[4 * S]) {
     if (begin >= end) return;
+    const Meta first = ld.meta8(begin, begin, lane);
     // An opaque definition keeps the mask in one VGPR for the whole walk instead of a
     // rematerialised literal per use.
     unsigned keep;
@@ -762,18 +834,16 @@ __device__ __forceinline__ void walkTask(const Ld& ld, const unsigned* offsets, 
     TaskWalk w{offsets, begin, end, lane, lds, 0u, keep, mh};
     auto clipLo = [&](unsigned t) { return max(offsets[t], begin); };
     auto clipHi = [&](unsigned t) { return min(offsets[t], end); };
-    walkPanels<0, S>(ld, w, clipLo(1), clipHi(2), acc);
-    walkPanels<1, S>(ld, w, clipLo(2), clipHi(3), acc);
-    walkPanels<2, S>(ld, w, clipLo(3), clipHi(4), acc);
-    walkPanels<3, S>(ld, w, clipLo(4), clipHi(5), acc);
-    walkPanels<kShared, S>(ld, w, clipLo(5), clipHi(16), acc);
+    const GroupBounds bounds{offsets[2], offsets[3], offsets[4]};
+    walkPanels<false, S>(ld, w, bounds, clipLo(1), clipHi(5), first, acc);
+    walkPanels<true, S>(ld, w, bounds, clipLo(5), clipHi(16), first, acc);
     waveSync();
 #pragma unroll 1
     for (unsigned i = 0; i < w.redoCount; ++i) {
         const unsigned panel = begin + __builtin_amdgcn_readfirstlane(lds.redo[i]);
         const unsigned groups = groupsOf(offsets, panel);
         Stage st;
-        loadStage<kShared, S>(ld, ld.meta8(panel, lane), groups, lane, st);
+        loadStage<true, S>(ld, ld.meta8(panel, panel, lane), RowBit{}, groups, lane, st);
         computePanelF32<Ld::kWide, S>(st, groups, lane, lds, acc);
     }
 }
@@ -805,28 +875,29 @@ __device__ __forceinline__ f32x4 load4(const float* p) {
     else return f32x4{p[0], p[1], p[2], p[3]};
 }
 
-// Store row `row` (lane & 31) of the accumulators: per tile i the lane holds the 16 features
-// 16 (2i + h) .. + 15 of the slice, block b / register 4i + j holding feature 2j + (b >> 1) +
-// 8 (b & 1) of that tile.
-template <bool Vec4>
-__device__ __forceinline__ void storeRow(const f32x16 (&acc)[4], float* rowBase, unsigned h,
-                                         bool nontemporal) {
+// Quad q (four consecutive features) of part i of the accumulators of one slice: per part the lane
+// holds the 16 features 16 (2i + h) .. + 15 of its row (lane & 31), block b / register 4i + j
+// holding feature 2j + (b >> 1) + 8 (b & 1) of them.
+template <unsigned I, unsigned Q>
+__device__ __forceinline__ f32x4 partQuad(const f32x16 (&acc)[4]) {
+    f32x4 v;
 #pragma unroll
-    for (unsigned i = 0; i < 4; ++i) {
-        float* dst = rowBase + 16 * (2 * i + h);
-#pragma unroll
-        for (unsigned q = 0; q < 4; ++q) {
-            f32x4 v;
-#pragma unroll
-            for (unsigned t = 0; t < 4; ++t) {
-                const unsigned o = 4 * q + t;
-                const unsigned hiHalf = o >= 8 ? 1u : 0u;
-                const unsigned rem = o - 8 * hiHalf;
-                v[t] = acc[(rem & 1u) * 2 + hiHalf][4 * i + (rem >> 1)];
-            }
-            store4<Vec4>(dst + 4 * q, v, nontemporal);
-        }
+    for (unsigned t = 0; t < 4; ++t) {
+        const unsigned o = 4 * Q + t;
+        const unsigned hiHalf = o >= 8 ? 1u : 0u;
+        const unsigned rem = o - 8 * hiHalf;
+        v[t] = acc[(rem & 1u) * 2 + hiHalf][4 * I + (rem >> 1)];
     }
+    return v;
+}
+
+template <class F, unsigned... I>
+__device__ __forceinline__ void forEachIndex(std::integer_sequence<unsigned, I...>, F f) {
+    (f(std::integral_constant<unsigned, I>{}), ...);
+}
+template <unsigned N, class F>
+__device__ __forceinline__ void forEachIndex(F f) {
+    forEachIndex(std::make_integer_sequence<unsigned, N>{}, f);
 }
 
 // Workgroup -> task. Workgroups are dispatched to the 8 XCDs round-robin by id, and XCD x walks
@@ -855,45 +926,47 @@ __device__ __forceinline__ unsigned equalBound(unsigned tasks, unsigned x) {
 // end anyway, so the order inside it leaves the L2 sharing of the in-order walk in place.
 constexpr unsigned kTailWindow = 512;
 
-__device__ __forceinline__ unsigned sizeClass(const Sw32Task* tasks, unsigned t) {
-    const unsigned p = tasks[t].end - tasks[t].begin;
-    return unsigned(p >= 96) + unsigned(p >= 192) + unsigned(p >= 288);
-}
-
 // Task at position r (r < n <= kTailWindow) of the window [w0, w0 + n) in size-class order. One
-// wave, all lanes active; every wave computes the same permutation of the window. The classes of
-// the window's tasks are loaded once (lane L: tasks L, L + 64, ...; all loads in flight together),
-// kept two bits per task in registers, and both passes below work on those.
+// wave, all lanes active; every wave computes the same permutation of the window. The sizes of the
+// window's tasks are loaded once (lane L: tasks L, L + 64, ...; all loads in flight together); per 64
+// tasks three compares give the wave masks of the tasks of at least 96, 192 and 288 panels, and
+// counting and picking are scalar work on those (two bits per task in a register and a ballot per
+// class took 3-4 us instead of about 2, half of it VALU work beside the other waves').
 __device__ __forceinline__ unsigned tailTask(const Sw32Task* tasks, unsigned w0, unsigned n,
                                              unsigned r, unsigned lane) {
-    constexpr unsigned kChunks = kTailWindow / kWave, kWords = (kChunks + 15) / 16;
-    unsigned bits[kWords] = {};
-#pragma unroll
-    for (unsigned ch = 0; ch < kChunks; ++ch)
-        bits[ch / 16] |= sizeClass(tasks, w0 + min(ch * kWave + lane, n - 1)) << (2 * (ch % 16));
-    auto member = [&](unsigned ch, unsigned c) {
-        return ch * kWave + lane < n && ((bits[ch / 16] >> (2 * (ch % 16))) & 3u) == c;
-    };
-    unsigned counts[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (unsigned ch = 0; ch < kChunks; ++ch)
-#pragma unroll
-        for (unsigned c = 0; c < 4; ++c)
-            counts[c] += unsigned(__builtin_popcountll(__builtin_amdgcn_ballot_w64(member(ch, c))));
-    unsigned c = 3, k = r;
-    while (c > 0 && k >= counts[c]) {
-        k -= counts[c];
-        --c;
-    }
+    constexpr unsigned kChunks = kTailWindow / kWave;
+    unsigned panels[kChunks];
 #pragma unroll
     for (unsigned ch = 0; ch < kChunks; ++ch) {
-        const bool in = member(ch, c);
-        const std::uint64_t mask = __builtin_amdgcn_ballot_w64(in);
+        const Sw32Task& t = tasks[w0 + min(ch * kWave + lane, n - 1)];
+        panels[ch] = t.end - t.begin;
+    }
+    std::uint64_t atLeast[kChunks][4]; // class c or above: c = 0 any task of the window
+    unsigned counts[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (unsigned ch = 0; ch < kChunks; ++ch) {
+        const unsigned in = n > ch * kWave ? min(n - ch * kWave, kWave) : 0u;
+        atLeast[ch][0] = in == kWave ? ~std::uint64_t(0) : (std::uint64_t(1) << in) - 1;
+#pragma unroll
+        for (unsigned c = 1; c < 4; ++c)
+            atLeast[ch][c] = __builtin_amdgcn_ballot_w64(panels[ch] >= 96 * c) & atLeast[ch][0];
+#pragma unroll
+        for (unsigned c = 0; c < 4; ++c) counts[c] += unsigned(__builtin_popcountll(atLeast[ch][c]));
+    }
+    // counts[c]: tasks of class c or above; position r is in the highest class whose count exceeds it.
+    const unsigned c = r < counts[3] ? 3u : r < counts[2] ? 2u : r < counts[1] ? 1u : 0u;
+    unsigned k = r - (c == 3 ? 0u : c == 2 ? counts[3] : c == 1 ? counts[2] : counts[1]);
+#pragma unroll
+    for (unsigned ch = 0; ch < kChunks; ++ch) {
+        const std::uint64_t mask = c == 3   ? atLeast[ch][3]
+                                   : c == 2 ? atLeast[ch][2] & ~atLeast[ch][3]
+                                   : c == 1 ? atLeast[ch][1] & ~atLeast[ch][2]
+                                            : atLeast[ch][0] & ~atLeast[ch][1];
         const unsigned count = unsigned(__builtin_popcountll(mask));
         if (k < count) {
             const unsigned below = __builtin_amdgcn_mbcnt_hi(unsigned(mask >> 32),
                                                              __builtin_amdgcn_mbcnt_lo(unsigned(mask), 0u));
-            const std::uint64_t hit = __builtin_amdgcn_ballot_w64(in && below == k);
+            const std::uint64_t hit = __builtin_amdgcn_ballot_w64(below == k) & mask;
             return w0 + ch * kWave + unsigned(__builtin_ctzll(hit));
         }
         k -= count;
@@ -901,37 +974,54 @@ __device__ __forceinline__ unsigned tailTask(const Sw32Task* tasks, unsigned w0,
     return w0 + r; // not reached: the window holds n tasks
 }
 
-// Boundaries x and x + 1 of the panel-balanced ranges: the first task starting at or past k/8 of
-// the panels, measured from the first task's begin (k = x, x + 1; `count` when none does; a view
-// over a later part of a plan's task list starts past panel 0). Lanes 32h .. 32h + 31 search boundary x + h
-// together: each step probes 32 evenly spaced tasks of the half's interval [l, r] (task r is known
-// to qualify; r = count stands for past the end) and keeps the stretch between the last probe
-// below the target and the first one at or past it, so a search takes about log32(T) dependent
-// loads instead of log2(T). Returns the boundary of each lane's half.
-__device__ __forceinline__ unsigned panelBound(const Sw32Task* tasks, unsigned count,
-                                               unsigned first, std::uint64_t panels, unsigned x,
-                                               unsigned lane) {
-    const unsigned h = lane >> 5, j = lane & 31;
-    const unsigned target = first + unsigned(panels * (x + h) / 8);
-    unsigned l = 0, r = count;
-    while (__builtin_amdgcn_ballot_w64(l < r) != 0) {
-        const unsigned stride = (r - l + 31) / 32; // 32 probes cover [l, r): r - l <= 32 stride
-        const unsigned q = l + j * stride;
-        const bool at = q >= r || tasks[min(q, count - 1)].begin >= target;
-        const unsigned half = unsigned(__builtin_amdgcn_ballot_w64(at) >> (32 * h));
-        const unsigned first = half ? unsigned(__builtin_ctz(half)) : 32u;
-        const unsigned nl = first == 0 ? l : l + (first - 1) * stride + 1;
-        r = first < 32 ? min(l + first * stride, r) : r;
-        l = nl;
+// Search for the boundary of a panel-balanced range: the first task of [l, r) that begins at or past
+// `target`, or r. Each step probes 64 evenly spaced tasks with one load (load(), apart from the
+// step that uses it, so that several searches' loads and other loads are in flight together) and
+// keeps the stretch between the last probe below the target and the first one at or past it: two
+// steps for the ranges of plans of up to 65,536 tasks. All bounds are wave-uniform.
+struct BoundSearch {
+    unsigned l, r, probed;
+    __device__ unsigned stride() const { return (r - l + kWave - 1) / kWave; }
+    __device__ bool done() const { return l >= r; }
+    __device__ void load(const Sw32Task* tasks, unsigned lane) {
+        if (!done()) probed = tasks[min(l + lane * stride(), r - 1)].begin;
     }
-    return l;
-}
+    __device__ void step(unsigned target, unsigned lane) {
+        if (done()) return;
+        const unsigned s = stride();
+        const std::uint64_t at =
+            __builtin_amdgcn_ballot_w64(l + lane * s >= r || probed >= target);
+        const unsigned first = at ? unsigned(__builtin_ctzll(at)) : kWave;
+        const unsigned nr = first < kWave ? min(l + first * s, r) : r;
+        if (first) l += (first - 1) * s + 1;
+        r = nr;
+    }
+};
 
 // Returns false when the workgroup has no task.
 __device__ __forceinline__ bool xcdTask(const KernelArgs& a, unsigned bid, unsigned& task) {
     const Sw32Task* tasks = a.m.tasks;
     const unsigned count = a.m.taskCount, x = bid & 7u, j = bid >> 3;
     const unsigned lane = threadIdx.x & (kWave - 1);
+    unsigned lo = equalBound(count, x), hi = equalBound(count, x + 1);
+    // Every workgroup starts at once and a quarter of the wave slots stays free: neither the order nor
+    // the balance decides anything, and finding them takes about 2 us of dependent loads (313 tasks of
+    // 8 waves, F128: 18.3 -> 16.2 us). With the slots nearly full they do matter: three skewed plans of
+    // 450 tasks ran 8-14% slower without them.
+    if (a.resident) {
+        task = lo + j;
+        return task < hi;
+    }
+    // Boundary k (0 < k < 8) of the balanced ranges lies within `reach` tasks of the equal-count one.
+    const unsigned reach = spareWorkgroups(count) / 2;
+    auto search = [&](unsigned k) {
+        const unsigned eq = equalBound(count, k);
+        const bool fixed = k == 0 || k == 8;
+        return BoundSearch{fixed ? eq : eq > reach ? eq - reach : 0u, fixed ? eq : eq + reach, 0u};
+    };
+    BoundSearch left = search(x), right = search(x + 1);
+    left.load(tasks, lane); // in flight beside the loads of the range check
+    right.load(tasks, lane);
     auto beginOf = [&](unsigned t) { return t < count ? tasks[t].begin : tasks[count - 1].end; };
     unsigned first[9];
     unsigned maxPanels = 0;
@@ -940,14 +1030,19 @@ __device__ __forceinline__ bool xcdTask(const KernelArgs& a, unsigned bid, unsig
 #pragma unroll
     for (unsigned k = 0; k < 8; ++k) maxPanels = max(maxPanels, first[k + 1] - first[k]);
     const std::uint64_t panels = first[8] - first[0];
-    unsigned lo = equalBound(count, x), hi = equalBound(count, x + 1);
     if (std::uint64_t(maxPanels) * 8 * 100 > panels * 103) {
-        const unsigned reach = spareWorkgroups(count) / 2;
-        const unsigned searched = panelBound(tasks, count, first[0], panels, x, lane);
-        const unsigned k = x + (lane >> 5), eq = equalBound(count, k);
-        const unsigned b = (k == 0 || k == 8) ? eq : min(max(searched, eq > reach ? eq - reach : 0u), eq + reach);
-        lo = __builtin_amdgcn_readlane(b, 0);
-        hi = __builtin_amdgcn_readlane(b, 32);
+        const unsigned targetLeft = first[0] + unsigned(panels * x / 8);
+        const unsigned targetRight = first[0] + unsigned(panels * (x + 1) / 8);
+        left.step(targetLeft, lane);
+        right.step(targetRight, lane);
+        while (!left.done() || !right.done()) {
+            left.load(tasks, lane);
+            right.load(tasks, lane);
+            left.step(targetLeft, lane);
+            right.step(targetRight, lane);
+        }
+        lo = left.l;
+        hi = right.l;
     }
     task = lo + j;
     if (task >= hi) return false;
@@ -963,14 +1058,15 @@ __device__ __forceinline__ bool xcdTask(const KernelArgs& a, unsigned bid, unsig
 // lane, broadcast by readlane), and the loads of kMergeBatch tiles are issued before they are added
 // in order, so a merge of many chunks waits for one load latency per batch, not per tile. Per element
 // the additions run in partialIds order whatever the batch, so Y is bitwise the same for any batch.
+// The task's waves take the row groups in turn.
 template <unsigned Features, bool Vec4>
 __device__ __forceinline__ void mergeSlice(const KernelArgs& a, const Sw32Task& task, unsigned k,
-                                           unsigned lane) {
+                                           unsigned wave, unsigned waves, unsigned lane) {
     constexpr unsigned kMergeBatch = 4;
     const unsigned sw = task.sw;
     const unsigned mrow = lane >> 3, mcol = k * kSlice + (lane & 7) * 4;
 #pragma unroll 1
-    for (unsigned g = 0; g < 4; ++g) {
+    for (unsigned g = wave; g < 4; g += waves) {
         const Sw32ReduceRange red = a.m.reductions[task.reduceFirst + g];
         const unsigned row0 = sw * 32 + g * 8;
         if (row0 >= a.rows) continue;
@@ -1014,109 +1110,138 @@ __device__ __forceinline__ void mergeSlice(const KernelArgs& a, const Sw32Task& 
     }
 }
 
-// One task over all S = Features / 128 slices of its SW, by `Waves` waves of one workgroup. With
-// more than one wave, wave w walks the w-th of `Waves` equal shares of the task's panels (its own
-// LDS tables, the same walk as a whole task), then hands its accumulators to wave 0, which adds them
-// in wave order and finishes the task alone. A task then takes about 1/Waves of the time, which
-// shortens launches whose longest tasks set the time (few tasks per wave slot).
+// LDS of one wave's walk.
+template <unsigned S>
+struct WaveLds {
+    static constexpr unsigned kAreas = S == 1 ? 1 : 2; // F256 computes its panels in pairs
+    alignas(16) _Float16 table16[256 * kAreas];
+    alignas(16) float table32[256];
+    alignas(16) u32x4 xtile[kAreas * 64 * S];
+    alignas(16) float mant[8 * kAreas];
+    alignas(16) unsigned short redo[384];
+};
+
+// The write-back of a task: the doubled sum of its waves, one or two parts (32 features each, 16 per lane
+// half) at a time. Every wave puts its part into LDS; then each (part, row group) of the round is one
+// wave's: lane L adds piece L & 7 (four features) of row 8g + (L >> 3) over the waves in order and
+// stores it, eight lanes to a 128-byte line of a row. `store(k, g, r, column, v)` stores four
+// features from `column` of slice k, row r of row group g. A single wave goes the same way, for the
+// stores: straight from the accumulators each instruction wrote 16 bytes of 64 different lines, and
+// a line of Y took eight of them (2.45M rows: F128 2,954 -> 2,854 us, F256 4,967 -> 4,851; 1M rows with
+// 64 hub rows, F256: 1,909 -> 1,774 us).
+//
+// LDS: [wave][part of the round][piece 0..7][33 x 16 bytes]: piece 2q + h of row r at index r, 33 so
+// that the eight pieces of a row fall into different banks.
+constexpr unsigned kPiece = 33, kPart = 8 * kPiece;
+template <unsigned Waves>
+constexpr unsigned kRoundParts = Waves == 1 ? 1 : 2;
+
+template <unsigned Waves>
+__device__ __forceinline__ void taskSync() {
+    if constexpr (Waves > 1)
+        __syncthreads();
+    else
+        waveSync();
+}
+
+template <unsigned S, unsigned Waves, class Store>
+__device__ __forceinline__ void writeTask(const f32x16 (&acc)[4 * S], f32x4* mem, unsigned wave,
+                                          unsigned lane, Store store) {
+    constexpr unsigned kParts = kRoundParts<Waves>;
+    const unsigned row = lane & 31, h = lane >> 5;
+    forEachIndex<4 * S / kParts>([&](auto round) __attribute__((always_inline)) {
+        constexpr unsigned kFirst = decltype(round)::value * kParts;
+        taskSync<Waves>(); // the walks' LDS, or the last round's, is no longer read
+        f32x4* mine = mem + wave * kParts * kPart;
+        forEachIndex<kParts * 4>([&](auto c) __attribute__((always_inline)) {
+            constexpr unsigned P = decltype(c)::value / 4, Q = decltype(c)::value % 4;
+            constexpr unsigned K = (kFirst + P) / 4, I = (kFirst + P) % 4;
+            const auto& slice = *reinterpret_cast<const f32x16(*)[4]>(&acc[4 * K]);
+            mine[P * kPart + (2 * Q + h) * kPiece + row] = partQuad<I, Q>(slice);
+        });
+        taskSync<Waves>();
+#pragma unroll 1
+        for (unsigned o = wave; o < 4 * kParts; o += Waves) {
+            const unsigned part = o >> 2, g = o & 3, r = lane >> 3, piece = lane & 7;
+            const f32x4* from = mem + part * kPart + ((piece & 3) * 2 + (piece >> 2)) * kPiece + 8 * g + r;
+            f32x4 sum = from[0];
+#pragma unroll
+            for (unsigned v = 1; v < Waves; ++v) sum += from[v * kParts * kPart];
+            sum *= 2.0f; // Y / 2 to Y, exact
+            const unsigned at = kFirst + part; // slice at / 4, features 32 (at % 4) .. + 31
+            store(at >> 2, g, r, 32 * (at & 3) + 4 * piece, sum);
+        }
+    });
+}
+
+// One task over all S = Features / 128 slices of its SW, by `Waves` waves of one workgroup:
+// wave w walks the w-th equal share of the task's panels (its own LDS tables, the same walk as a whole
+// task), and their sum, in wave order, is written by all of them (writeTask). A task then takes about
+// 1/waves of the time, which shortens launches whose longest tasks set the time (few tasks per wave
+// slot).
 template <unsigned Features, unsigned Addr, unsigned Waves = 1>
 __device__ __forceinline__ void runTask(const KernelArgs& a, unsigned taskIndex) {
     constexpr unsigned S = Features / kSlice;
-    constexpr unsigned kAreas = S == 1 ? 1 : 2; // F256 computes its panels in pairs
-    __shared__ __align__(16) _Float16 table16[Waves][256 * kAreas];
-    __shared__ __align__(16) float table32[Waves][256];
-    __shared__ __align__(16) u32x4 xtile[Waves][kAreas * 64 * S];
-    __shared__ __align__(16) float mant[Waves][8 * kAreas];
-    __shared__ unsigned short redo[Waves][384];
+    constexpr std::size_t kWalkBytes = sizeof(WaveLds<S>) * Waves;
+    constexpr std::size_t kWriteBytes = std::size_t(Waves) * kRoundParts<Waves> * kPart * 16;
+    __shared__ __align__(16) unsigned char shared[kWalkBytes > kWriteBytes ? kWalkBytes : kWriteBytes];
     __shared__ unsigned lastFlag[S];
     const unsigned wave = Waves == 1 ? 0u : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const unsigned lane = Waves == 1 ? threadIdx.x : threadIdx.x & 63u;
     const Sw32Task task = a.m.tasks[taskIndex];
     const unsigned sw = task.sw;
-    const Loader<Addr> ld(a, task.begin, task.end, Features);
-    const Lds lds{table16[wave], table32[wave], xtile[wave], mant[wave], redo[wave]};
-
-    f32x16 acc[4 * S];
-#pragma unroll
-    for (unsigned b = 0; b < 4 * S; ++b) acc[b] = f32x16{};
     unsigned lo = task.begin, hi = task.end;
     if constexpr (Waves > 1) {
         const std::uint64_t n = hi - lo;
         lo = task.begin + unsigned(n * wave / Waves);
         hi = task.begin + unsigned(n * (wave + 1) / Waves);
     }
-    walkTask<S>(ld, a.m.bucketOffsets + std::size_t(sw) * 17, lo, hi, lane, lds, acc);
-#pragma unroll
-    for (unsigned b = 0; b < 4 * S; ++b) acc[b] *= 2.0f; // Y / 2 to Y, exact
-    if constexpr (Waves > 1) {
-        // One accumulator block (16 floats per lane) per round, as four 16-byte chunks per lane
-        // laid out chunk-major so that each chunk's 64 lanes are contiguous.
-        __shared__ __align__(16) f32x4 handoff[Waves - 1][4][kWave];
-#pragma unroll
-        for (unsigned b = 0; b < 4 * S; ++b) {
-            if (wave != 0) {
-#pragma unroll
-                for (unsigned q = 0; q < 4; ++q)
-                    handoff[wave - 1][q][lane] =
-                        f32x4{acc[b][4 * q], acc[b][4 * q + 1], acc[b][4 * q + 2], acc[b][4 * q + 3]};
-            }
-            __syncthreads();
-            if (wave == 0) {
-#pragma unroll
-                for (unsigned v = 0; v + 1 < Waves; ++v)
-#pragma unroll
-                    for (unsigned q = 0; q < 4; ++q) {
-                        const f32x4 o = handoff[v][q][lane];
-#pragma unroll
-                        for (unsigned e = 0; e < 4; ++e) acc[b][4 * q + e] += o[e];
-                    }
-            }
-            __syncthreads();
-        }
-        if (wave != 0) return;
-    }
+    Loader<Addr> ld(a, lo, hi, Features);
+    WaveLds<S>& mem = reinterpret_cast<WaveLds<S>*>(shared)[wave];
+    const Lds lds{mem.table16, mem.table32, mem.xtile, mem.mant, mem.redo};
 
-    const unsigned row = lane & 31, h = lane >> 5;
+    f32x16 acc[4 * S];
+#pragma unroll
+    for (unsigned b = 0; b < 4 * S; ++b) acc[b] = f32x16{};
+    walkTask<S>(ld, a.m.bucketOffsets + std::size_t(sw) * 17, lo, hi, lane, lds, acc);
+    // The last MFMAs' results are not interlocked against the moves that read them, and the compiler
+    // has padded a path into this point with fewer wait states than the 18 they need.
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15\n\ts_nop 1");
+    __builtin_amdgcn_sched_barrier(0);
+
     // Write-back. An unsplit task stores its rows of Y (nontemporal: nothing reads them again in this
-    // launch); a split task stores the row groups of task.mask as 8-row partial tiles. One store site
-    // for both, so that the accumulators are dead once it is passed.
+    // launch); a split task stores the row groups of task.mask as 8-row partial tiles.
     const bool split = task.partial != kNoPartial;
-    const unsigned rw = row >> 3;
-    float* dst;
-    bool mine;
-    if (!split) {
-        const unsigned r = sw * 32 + row;
-        mine = r < a.rows;
-        dst = a.y + std::size_t(r) * Features;
-    } else {
-        mine = (task.mask >> rw) & 1u;
-        const std::size_t tile = task.partial + __popc(task.mask & ((1u << rw) - 1u));
-        dst = a.partials + (tile * 8 + (row & 7)) * Features;
-    }
-    auto sub = [&](unsigned k) -> const f32x16(&)[4] {
-        return *reinterpret_cast<const f32x16(*)[4]>(&acc[4 * k]);
-    };
-    if (mine) {
-        if (a.vec4) {
-#pragma unroll
-            for (unsigned k = 0; k < S; ++k) storeRow<true>(sub(k), dst + k * kSlice, h, !split);
-        } else {
-#pragma unroll
-            for (unsigned k = 0; k < S; ++k) storeRow<false>(sub(k), dst + k * kSlice, h, !split);
-        }
-    }
+    writeTask<S, Waves>(
+        acc, reinterpret_cast<f32x4*>(shared), wave, lane,
+        [&](unsigned k, unsigned g, unsigned r, unsigned column, const f32x4& v) {
+            float* dst;
+            if (!split) {
+                const unsigned row = sw * 32 + 8 * g + r;
+                if (row >= a.rows) return;
+                dst = a.y + std::size_t(row) * Features;
+            } else {
+                if (!((task.mask >> g) & 1u)) return;
+                const std::size_t tile = task.partial + __popc(task.mask & ((1u << g) - 1u));
+                dst = a.partials + (tile * 8 + r) * Features;
+            }
+            if (a.vec4)
+                store4<true>(dst + k * kSlice + column, v, !split);
+            else
+                store4<false>(dst + k * kSlice + column, v, !split);
+        });
     if (!split) return;
 
     // Completion tickets, one per slice: the release fence at agent scope publishes this task's
-    // partial tiles before its tickets, and the acquire fence of a last arriver makes every other
+    // partial tiles before its tickets, and the acquire fence of the last arriver makes every other
     // task's tiles visible (the XCD L2s are not coherent with each other, so the release writes back
-    // and the acquire invalidates). Both work on the whole L2 of the XCD and cost every wave that runs
-    // there, so there is one release for all slices, and an acquire only where tiles are read. With an
-    // acq_rel ticket per slice instead, every split task invalidated its L2 once per slice (F256,
-    // 1M rows with 64 hub rows, 7,200 split tasks: 2,435 -> 1,923 us; a 262K-row power-law graph:
-    // 441 -> 401 us; 2.45M rows: 5,125 -> 5,005 us; F128, one ticket per task: no change).
-    waveSync();
-    if (lane == 0) {
+    // and the acquire invalidates). One release for all slices, and an acquire only where tiles are
+    // read: both work on the whole L2 of the XCD. With several waves, each one's stores have reached
+    // that L2 (vmcnt 0) before the barrier in front of the release.
+    if constexpr (Waves > 1) __builtin_amdgcn_s_waitcnt(0x0F70); // vmcnt(0)
+    taskSync<Waves>();
+    if (wave == 0 && lane == 0) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
 #pragma unroll
         for (unsigned k = 0; k < S; ++k) {
@@ -1126,15 +1251,15 @@ __device__ __forceinline__ void runTask(const KernelArgs& a, unsigned taskIndex)
             lastFlag[k] = ticket == task.chunks - 1;
         }
     }
-    waveSync();
+    taskSync<Waves>();
 #pragma unroll 1
     for (unsigned k = 0; k < S; ++k) {
         if (!lastFlag[k]) continue;
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         if (a.vec4)
-            mergeSlice<Features, true>(a, task, k, lane);
+            mergeSlice<Features, true>(a, task, k, wave, Waves, lane);
         else
-            mergeSlice<Features, false>(a, task, k, lane);
+            mergeSlice<Features, false>(a, task, k, wave, Waves, lane);
     }
 }
 
@@ -1221,52 +1346,81 @@ int currentDeviceCus() {
     return cus;
 }
 
-// Waves per task: 2 when the plan has few tasks for the chip's wave slots, so that the longest
-// tasks, not the bandwidth, set the launch time; else 1. Measured crossovers on MI355X (256 CUs;
-// wave slots = CUs x 4 SIMDs x the kernel's waves per SIMD, 4 at F128 and 2 at F256): F128 gains
-// below about 3 tasks per slot (-39% at 250 tasks, -6% at 8,790, even at 12,500, +3% at 38,281),
-// F256 below about half a task per slot (-26% at 1,000 tasks, +1% at 1,875).
-unsigned taskWaves(unsigned taskCount, unsigned features) {
-    if (const unsigned forced = forcedWaves.load()) return forced;
+// Wave slots of the current device: CUs x 4 SIMDs x the kernel's waves per SIMD, 4 at F128 and 2 at
+// F256 (0 when unknown).
+std::uint64_t waveSlots(unsigned features) {
     const int cus = currentDeviceCus();
-    if (cus <= 0) return 1;
-    const std::uint64_t slots = std::uint64_t(cus) * 4 * (features == 128 ? 4 : 2);
-    const std::uint64_t limit = features == 128 ? 3 * slots : slots / 2;
-    return taskCount < limit ? 2u : 1u;
+    return cus <= 0 ? 0 : std::uint64_t(cus) * 4 * (features == 128 ? 4 : 2);
+}
+
+// Waves per task. Few tasks for the chip: as many waves as keep the chip's slots in use, since the
+// longest tasks, not the bandwidth, set the launch time. Measured on MI355X (us; 256 CUs, 4,096 wave slots at
+// F128 and 2,048 at F256; matrices of 20 or 32 entries per row with power-law tails, 8 uniform where
+// marked u: short tasks, to which more waves are of least use):
+//
+//   tasks        250   500u   651  1,002 1,000u 2,090  3,135 4,251  8,566 25,076 31,250u 38,196 78,036
+//   F128 1 wave   79   18.9   129    123   20.6   154    152   159    270    490     345  1,147  2,854
+//        2        45   12.6    74     72   15.6    94     76   113    223    461     354  1,133  2,897
+//        4        27   10.6    50     41   14.9    65     74   118    241    545     394  1,182  3,126
+//        8        20   10.8    36     40   22.7    80    105   160    332
+//   F256 1        99   25.2   161    154   27.0   180    169   197    377    784     599  1,774  4,851
+//        2        56   18.8    97     95   22.6   111    116   190    382    849     627  1,767  5,105
+//        4        34   16.3    56     57   29.9   113    144   224    462  1,127     796  1,966  5,708
+//        8        27   24.3    66     74   43.9   164    223   346    711
+//
+// The lines: 8 waves while every wave has a slot (slots / 8 tasks), 4 up to 3/4 slots; then 2 up to
+// 8 tasks per slot at F128 and 4 at F256, where one wave per task has longer walks and fewer fills.
+unsigned taskWaves(unsigned taskCount, unsigned features, std::uint64_t slots) {
+    if (const unsigned forced = forcedWaves.load()) return forced;
+    if (!slots) return 1;
+    const std::uint64_t tasks = taskCount;
+    if (8 * tasks <= slots) return 8;
+    if (4 * tasks <= 3 * slots) return 4;
+    return tasks <= (features == 128 ? 8 : 4) * slots ? 2u : 1u;
 }
 
 template <unsigned Features>
-void launch(const KernelArgs& args, hipStream_t stream) {
+void launch(KernelArgs args, hipStream_t stream) {
     // Buffer addressing needs the packed X and the scales within 32-bit byte offsets, with room for
     // the padding sentinel to land out of range, and 16-byte aligned X tiles. A packed X that is
     // only u16-aligned takes the 64-bit instance with 2-byte tile loads. setSpmmLaunchOverrides
     // can select the 64-bit instance for any size (used by the tests).
     const bool misaligned = reinterpret_cast<std::uintptr_t>(args.packedX) % 16 != 0;
     const bool wide = std::uint64_t(args.cols) * Features > 0xFFFFFF00ull || forcedWide.load();
-    const dim3 grid(args.m.taskCount + 8 * spareWorkgroups(args.m.taskCount), 1);
-    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kWave), 0, stream, args); };
-    auto go2 = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(2 * kWave), 0, stream, args);
+    const std::uint64_t slots = waveSlots(Features);
+    const unsigned waves = misaligned || wide ? 1u : taskWaves(args.m.taskCount, Features, slots);
+    args.resident = 4 * std::uint64_t(args.m.taskCount) * waves <= 3 * slots;
+    const dim3 grid(args.resident ? args.m.taskCount
+                                  : args.m.taskCount + 8 * spareWorkgroups(args.m.taskCount));
+    auto go = [&](auto kernel, unsigned n) {
+        hipLaunchKernelGGL(kernel, grid, dim3(n * kWave), 0, stream, args);
     };
-    const bool split = !misaligned && !wide && taskWaves(args.m.taskCount, Features) == 2;
     if constexpr (Features == 256) {
         if (misaligned)
-            go(spmmInt8Kernel256<kGlobalU16>);
+            go(spmmInt8Kernel256<kGlobalU16>, 1);
         else if (wide)
-            go(spmmInt8Kernel256<kGlobal>);
-        else if (split)
-            go2(spmmInt8Kernel256<kBuffer, 2>);
+            go(spmmInt8Kernel256<kGlobal>, 1);
+        else if (waves == 8)
+            go(spmmInt8Kernel256<kBuffer, 8>, 8);
+        else if (waves == 4)
+            go(spmmInt8Kernel256<kBuffer, 4>, 4);
+        else if (waves == 2)
+            go(spmmInt8Kernel256<kBuffer, 2>, 2);
         else
-            go(spmmInt8Kernel256<kBuffer>);
+            go(spmmInt8Kernel256<kBuffer>, 1);
     } else {
         if (misaligned)
-            go(spmmInt8Kernel128<kGlobalU16>);
+            go(spmmInt8Kernel128<kGlobalU16>, 1);
         else if (wide)
-            go(spmmInt8Kernel128<kGlobal>);
-        else if (split)
-            go2(spmmInt8Kernel128<kBuffer, 2>);
+            go(spmmInt8Kernel128<kGlobal>, 1);
+        else if (waves == 8)
+            go(spmmInt8Kernel128<kBuffer, 8>, 8);
+        else if (waves == 4)
+            go(spmmInt8Kernel128<kBuffer, 4>, 4);
+        else if (waves == 2)
+            go(spmmInt8Kernel128<kBuffer, 2>, 2);
         else
-            go(spmmInt8Kernel128<kBuffer>);
+            go(spmmInt8Kernel128<kBuffer>, 1);
     }
 }
 
@@ -1339,7 +1493,7 @@ void launchSpmmInt8(Sw32DeviceView matrix, const std::int8_t* packedX, const flo
     const bool vec4 = (reinterpret_cast<std::uintptr_t>(output) |
                        reinterpret_cast<std::uintptr_t>(workspace.partials)) % 16 == 0;
     KernelArgs args{matrix, packedX, scales, output, workspace.partials, workspace.counters,
-                    rows,   cols,    unsigned(vec4)};
+                    rows,   cols,    0u, unsigned(vec4)};
 #ifdef TCC_SPMM_TIMELINE
     args.stamps = timelineStamps(matrix.taskCount);
 #endif

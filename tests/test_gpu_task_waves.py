@@ -1,0 +1,55 @@
+"""Y at both sides of every line of the rule that picks a task's waves and its workgroup order.
+
+With `slots` wave slots, a plan takes 8 waves per task up to slots / 8 tasks, 4 up to 3/4 slots, and 2
+or 1 above; plans that fill at most half of the slots skip the range search and the tail window. Each
+plan here has short tasks of few panels (waves without any panel), split SWs (chunks merged by the
+workgroup's waves) and a last SW with missing rows.
+"""
+import numpy as np
+import pytest
+
+import tcc_spmm_amd as T
+from gpu_cases import ATOL, RTOL, features, gpu_prepare
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrix(tasks, rng):
+    """A matrix whose plan has exactly `tasks` tasks: SWs of a few panels and, among them, one row of
+    7,000 entries (876 panels, three tasks) per 400 tasks."""
+    hubs = max(1, tasks // 400)
+    sws = tasks - 2 * hubs
+    rows, cols = 32 * sws - 5, 9000
+    degree = rng.integers(0, 4, rows)
+    degree[rng.choice(sws, hubs, replace=False) * 32 + rng.integers(0, 27, hubs)] = 7000
+    lists = [np.sort(rng.choice(cols, d, replace=False)) if d else np.zeros(0, np.int64)
+             for d in degree]
+    off = np.concatenate([[0], np.cumsum(degree)]).astype(np.uint32)
+    src = np.concatenate(lists).astype(np.uint32)
+    val = rng.uniform(-1, 1, src.size).astype(np.float32)
+    return T.make_canonical_csr(rows, cols, off, src, val)
+
+
+@pytest.mark.parametrize("feats", [128, 256])
+@pytest.mark.parametrize("num,den,extra", [(1, 32, 0), (1, 16, 0), (1, 16, 1), (1, 8, 0), (1, 8, 1),
+                                           (3, 4, 0), (3, 4, 1)])
+def test_spmm_at_the_lines_of_the_waves_rule(oracle, gpu, feats, num, den, extra):
+    import torch
+    from tcc_spmm_amd.device import TorchDeviceMatrix
+    slots = torch.cuda.get_device_properties(gpu).multi_processor_count * 4 * (4 if feats == 128 else 2)
+    tasks = slots * num // den + extra
+    csr = _matrix(tasks, np.random.default_rng(tasks + feats))
+    fmt = T.convert_csr_to_sw32(csr.rows, csr.cols, csr)
+    assert len(fmt.tasks) == tasks and fmt.partial_count > 0
+    packed, scale, _, sc, pk = gpu_prepare(features(csr.cols, feats, seed=tasks), gpu)
+    dm = TorchDeviceMatrix(fmt, feats, device=gpu)
+    y = torch.full((csr.rows, feats), float("nan"), device=gpu)
+    dm.partials.fill_(float("nan"))
+    for _ in range(2):  # the second launch finds the counters as the first left them
+        dm.spmm(packed, scale, y)
+    assert int(dm.counters.abs().sum()) == 0
+    ofmt = oracle.sw32(csr.rows, csr.cols, *csr.views())
+    # A sum of n FP32 additions of exact products is off by at most n * 2^-24 of the sum of their
+    # magnitudes; over the 7,000 terms of a hub row that is covered by the oracle's conditioned bound.
+    st = ofmt.check_full(pk, sc, y.cpu().numpy(), ATOL, RTOL, cond=16.0, threads=8)
+    assert st["checked"] == y.numel() and st["bad"] == 0, st

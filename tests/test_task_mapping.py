@@ -174,3 +174,56 @@ def test_offset_task_list_maps_like_the_whole(cfg):
     for shift in (int(sub[0]), int(sub[0]) + 12345):
         assert _bounds(sub - sub[0] + shift, end - int(sub[0]) + shift) == base
         assert _covered_once(sub - sub[0] + shift, end - int(sub[0]) + shift) == (True, True)
+
+
+def _bound_search(begin, l, r, target):
+    """BoundSearch: 64 probes per step over [l, r); returns the bound and the steps it took."""
+    steps = 0
+    while l < r:
+        stride = (r - l + WAVE - 1) // WAVE
+        at = [l + j * stride >= r or begin[min(l + j * stride, r - 1)] >= target
+              for j in range(WAVE)]
+        first = at.index(True) if True in at else WAVE
+        nr = min(l + first * stride, r) if first < WAVE else r
+        if first:
+            l += (first - 1) * stride + 1
+        r = nr
+        steps += 1
+    return l, steps
+
+
+def test_range_search_is_the_clamped_lower_bound():
+    """Searching only the stretch a boundary may move in, 64 probes at a time, gives the lower bound
+    over the whole list clamped to that stretch, in two steps for up to 65,536 tasks."""
+    rng = np.random.default_rng(6)
+    for n in list(range(8, 80, 5)) + [1000, 38281, 65536, 79199]:
+        for kind in ("random", "runs", "empty"):
+            sizes = {"random": rng.integers(0, 385, n), "empty": np.zeros(n, np.int64),
+                     "runs": np.where(rng.random(n) < 0.7, 0, rng.integers(1, 385, n))}[kind]
+            begin = np.concatenate([[0], np.cumsum(sizes)[:-1]]).astype(np.int64)
+            total, reach = int(sizes.sum()), _spare(n) // 2
+            for k in range(1, 8):
+                eq = _equal(n, k)
+                lo, hi = max(eq - reach, 0), eq + reach
+                assert hi <= n
+                for target in {0, total, total + 1, total * k // 8, int(begin[eq])}:
+                    want = min(max(int(np.searchsorted(begin, target, side="left")), lo), hi)
+                    got, steps = _bound_search(begin, lo, hi, target)
+                    assert got == want, (kind, n, k, target)
+                    assert steps <= (2 if n <= 65536 else 3)
+
+
+def test_tail_order_from_nested_masks():
+    """Counting tasks of at least 96, 192 and 288 panels and picking the k-th of a class from the
+    difference of two nested masks gives the stable order by descending class."""
+    rng = np.random.default_rng(7)
+    for n in (1, 2, 63, 64, 65, 130, 511, 512):
+        panels = rng.choice([0, 12, 95, 96, 191, 192, 287, 288, 384], n)
+        above = [panels >= 96 * c for c in range(4)]
+        counts = [int(a.sum()) for a in above]
+        order = []
+        for r in range(n):
+            c = next(c for c in (3, 2, 1, 0) if r < counts[c])
+            member = above[c] & ~above[c + 1] if c < 3 else above[c]
+            order.append(int(np.flatnonzero(member)[r - (counts[c + 1] if c < 3 else 0)]))
+        assert order == list(np.argsort(-_size_class(panels), kind="stable"))

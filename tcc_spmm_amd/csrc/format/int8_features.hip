@@ -2,8 +2,8 @@
 //
 // quantize: rows of features % 4 == 0 (16-byte aligned) use 16-byte loads of 4-feature groups and one
 // dword store per 4 quantized bytes: quantizeRowsFit for F <= 256 (one group per lane, several rows
-// per thread held in registers, X read once), quantizeRowsLong above; other rows one wave per row
-// (quantizeRows). The row's |x| maximum is reduced across its lanes with shuffles, and every element
+// per thread held in registers, X read once), quantizeRowsLong above; other widths (5 <= F <= 2048) go
+// through LDS a tile of rows at a time (quantizeTile), the rest one wave per row (quantizeRows). The row's |x| maximum is reduced across its lanes with shuffles, and every element
 // is divided by the scale with the IEEE-correct FP32 divide and rounded half-to-even. Results are bit-identical to reference
 // src/format/int8_quantize.cu:4-25.
 //
@@ -151,6 +151,60 @@ __global__ __launch_bounds__(256) void quantizeRowsLong(const f32x4* __restrict_
     }
 }
 
+// Rows of any width 5 <= F <= kTileFeatures whose X is 16-byte aligned, in tiles of kRows rows (a power
+// of two, at least 4, so that every tile starts 16-byte aligned in X and 4-byte aligned in q). A row of
+// a width that is not a multiple of 4 is not 16-byte aligned, but a tile is one contiguous stretch: it
+// is copied to LDS with 16-byte loads, the row maxima are taken there (256 / rows threads each), and q is
+// written four bytes at a time across the row ends. Bound by HBM: 300,007 x 50 (75 MB) in 49.9 us with
+// one wave per row and 4-byte loads, 18.7 us with tiles
+// (50,001 x 602: 48.8 -> 36.4; 1,000,003 x 5: 155 -> 8.5).
+constexpr unsigned kTileFeatures = 2048, kTileFloats = 4096;
+
+__global__ __launch_bounds__(256) void quantizeTile(const float* __restrict__ x,
+                                                     std::int8_t* __restrict__ q,
+                                                     float* __restrict__ scale, unsigned sources,
+                                                     unsigned features, unsigned rows,
+                                                     unsigned rowMagic) {
+    extern __shared__ __align__(16) float tile[]; // [rows x features], then the rows' scales + 1
+    const unsigned t = threadIdx.x;
+    const std::size_t row0 = std::size_t(blockIdx.x) * rows;
+    const unsigned live = unsigned(min(std::size_t(rows), sources - row0));
+    const unsigned n = live * features, quads = n / 4;
+    float* rowScale = tile + rows * features;
+    const float* xt = x + row0 * features;
+    for (unsigned i = t; i < quads; i += 256)
+        reinterpret_cast<f32x4*>(tile)[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(xt) + i);
+    for (unsigned i = 4 * quads + t; i < n; i += 256) tile[i] = xt[i];
+    __syncthreads();
+    const unsigned perRow = 256 / rows, row = t / perRow;
+    float m = 0.0f;
+    if (row < live)
+        for (unsigned j = t % perRow; j < features; j += perRow)
+            m = fmaxf(m, fabsf(tile[row * features + j]));
+    for (unsigned offset = perRow / 2; offset > 0; offset >>= 1) m = fmaxf(m, __shfl_xor(m, offset));
+    if (t % perRow == 0 && row < live) {
+        const float s = m == 0.0f ? 1.0f : m / 127.0f;
+        scale[row0 + row] = s;
+        rowScale[row] = s;
+    }
+    if (t == 0) rowScale[live] = 1.0f; // read beside the last row's, never used
+    __syncthreads();
+    std::int8_t* qt = q + row0 * features;
+    // floor(e / features) is the high word of e x rowMagic (floor(2^32 / features) + 1): e < 2^16 here.
+    for (unsigned i = t; i < quads; i += 256) {
+        const f32x4 v = reinterpret_cast<const f32x4*>(tile)[i];
+        const unsigned r = __umulhi(4 * i, rowMagic), left = (r + 1) * features - 4 * i;
+        const float s0 = rowScale[r], s1 = rowScale[r + 1];
+        unsigned qd = 0;
+#pragma unroll
+        for (unsigned j = 0; j < 4; ++j)
+            qd |= (unsigned(quantizeOne(v[j], j < left ? s0 : s1)) & 0xFFu) << (8 * j);
+        __builtin_nontemporal_store(qd, reinterpret_cast<unsigned*>(qt) + i);
+    }
+    for (unsigned i = 4 * quads + t; i < n; i += 256)
+        qt[i] = std::int8_t(quantizeOne(tile[i], rowScale[__umulhi(i, rowMagic)]));
+}
+
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // One thread per 16-byte tile; q is read once and packed written once, so both use nontemporal
@@ -183,14 +237,25 @@ __global__ __launch_bounds__(256) void packPairs(const std::uint8_t* __restrict_
 namespace {
 
 // The quantize kernels for one call: the vector kernels for 16-byte aligned rows of features % 4 ==
-// 0 with a 4-byte aligned output, the scalar kernel otherwise. `Packed` writes the packed16 layout
+// 0 with a 4-byte aligned output, the tile kernel for other widths of such buffers (at F < 5 four
+// features can span more than two rows; above 2,048 a tile does not fit LDS beside others), the scalar
+// kernel otherwise. `Packed` writes the packed16 layout
 // (features % 16 == 0, checked by the caller).
 template <bool Packed>
 void launchQuantize(const float* x, std::int8_t* out, float* scale, std::uint32_t sources,
                     std::uint32_t features, hipStream_t stream) {
-    const bool vector = features % 4 == 0 && reinterpret_cast<std::uintptr_t>(x) % 16 == 0 &&
-                        reinterpret_cast<std::uintptr_t>(out) % 4 == 0;
-    if (vector) {
+    const bool aligned = reinterpret_cast<std::uintptr_t>(x) % 16 == 0 &&
+                         reinterpret_cast<std::uintptr_t>(out) % 4 == 0;
+    if (!Packed && aligned && features % 4 != 0 && features >= 5 && features <= kTileFeatures) {
+        // Tiles of up to 16 KB, and small enough for a block per CU where there are few rows.
+        unsigned rows = 256;
+        while (rows > 4 && (rows * features > kTileFloats || sources / rows < 256)) rows /= 2;
+        const unsigned blocks = unsigned((std::size_t(sources) + rows - 1) / rows);
+        const std::size_t lds = (std::size_t(rows) * features + rows + 1) * sizeof(float);
+        const unsigned magic = unsigned((std::uint64_t(1) << 32) / features) + 1;
+        hipLaunchKernelGGL(quantizeTile, dim3(blocks), dim3(256), lds, stream, x, out, scale, sources,
+                           features, rows, magic);
+    } else if (aligned && features % 4 == 0) {
         const unsigned groups = features / 4;
         const auto* xv = reinterpret_cast<const f32x4*>(x);
         auto* qv = reinterpret_cast<unsigned*>(out);

@@ -5,24 +5,22 @@
 //   plans; each XCD walks a contiguous range of the task list (xcdTask), balanced by panels when skewed,
 //   the range's last 512 tasks longest size class first (tailTask).
 //   The wave walks the task's panels once, in order, and accumulates all 32 rows x F features of
-//   the SW: four v_mfma_f32_32x32x8_f16 per panel and 128-feature slice (one per 32-feature block;
-//   M = features, N = the 32 rows, K = the panel's 8 slots) into 4 x 16 FP32 accumulators per
-//   slice. F256 runs both slices in the same wave, so the A side of a panel is loaded and built
-//   once, and takes its panels in pairs: four v_mfma_f32_32x32x16_f16 per pair and slice, K = the
-//   pair's 16 slots. Plans with few tasks for the chip take two, four or eight waves per task instead
-//   (taskWaves), each walking its share of the panels; the write-back adds their accumulators (writeTask).
+//   the SW, two panels at a time: four v_mfma_f32_32x32x16_f16 per pair and 128-feature slice (one per
+//   32-feature block; M = features, N = the 32 rows, K = the pair's 16 slots) into 4 x 16 FP32
+//   accumulators per slice. F256 runs both slices in the same wave, so the A side of a pair is loaded
+//   and built once. Plans with few tasks for the chip take two, four or eight waves per task instead
+//   (taskWaves), each walking its share of the pairs; the write-back adds their accumulators (writeTask).
 //
-// Operands of one panel
-//   A (features x slots): the 8 slot rows of the X slice are gathered with one dwordx4 load per
-//   lane (lane L: 16-byte tile L & 7 of slot L >> 3) and stored to LDS as [slot][128 bytes].
-//   Lane l then reads dword l & 31 of slots 4h..4h+3 (h = l >> 5): byte b of that dword is block
-//   b's feature for M index l & 31, so each lane dequantizes 16 bytes (4 slots x 4 blocks), with
-//   the four slots' scale mantissas read from LDS as one 16-byte broadcast.
-//   B (slots x rows): an LDS table [32 rows][8 slots] of f16 A values; lane l reads row l & 31,
-//   slots 4h..4h+3. Rows of row groups the panel's bucket does not touch hold 0.
+// Operands of one pair (walkPairs; the 64-bit-addressed instances build the same ones in walkPanels)
+//   A (features x slots): the 8 slot rows of each panel's X slice are gathered with one 16-byte load per
+//   lane (lane L: 16-byte tile L & 7 of slot L >> 3) into LDS as [slot][128 bytes]. Lane l then reads
+//   dword l & 31 of slots 4h..4h+3 (h = l >> 5): byte b of that dword is block b's feature for M index
+//   l & 31, so each lane dequantizes 16 bytes (4 slots x 4 blocks) a panel, with the four slots' scale
+//   mantissas read from LDS as one 16-byte broadcast.
+//   B (slots x rows): an LDS table of f16 A values; lane l reads row l & 31, slots 4h..4h+3 of both
+//   panels. Rows of row groups a panel's bucket does not touch hold 0.
+//   Each operand takes its four values from the first panel and then four from the second.
 //   D: lane l holds row l & 31 and, per block, M indices 8i + 4h + j (register 4i + j).
-//   F256 pairs: both panels' X rows, mantissas and tables sit in two LDS areas, and each operand
-//   takes its four values from the first panel and then four from the second (K = 16).
 //
 // Exact TF32 products in f16. With the slot's scale written s = m * 2^e (m in [0.5, 1)),
 // x_hat = tf32(fp32(q * s)) = tf32(fp32(q * m)) * 2^e exactly whenever s is normal, and
@@ -38,10 +36,9 @@
 // is subnormal) takes an FP32 path with the same products: v_mfma_f32_32x32x2_f32 on tf32(a) / 2 and
 // the TF32 features. (Halving a value below 2^-125 rounds it, an error far below the tolerance.)
 //
-// The panels are walked by a software pipeline (F128: metadata two panels ahead, in pairs of panels,
-// A values and X one panel ahead; F256: metadata four panels ahead, A values and X two) whose memory
-// operations are identical on every path. F128
-// runs four waves per SIMD (128 registers each, accumulators included), F256 two (248 registers).
+// The walk is a software pipeline over pairs: metadata two pairs ahead, A values, scales and X one,
+// the X rows as loads to LDS. F128 runs four waves per SIMD (128 registers each, accumulators included),
+// F256 two.
 //
 // Split SWs (reference src/kernel/spmm_kernel.cuh:228-282): a split task stores its row groups of
 // `task.mask` as 8-row partial tiles [tile][8][F]; lane 0 then takes, per slice, an agent-scope
@@ -138,24 +135,11 @@ __device__ __forceinline__ unsigned lanePermute(unsigned v, unsigned srcLane) {
     return unsigned(__builtin_amdgcn_ds_bpermute(int(srcLane * 4), int(v)));
 }
 
-// Metadata of panels q and q + 1 loaded together (F128 walk): lane L holds slot L & 7 of panel
+// Metadata of panels q and q + 1 loaded together: lane L holds slot L & 7 of panel
 // q + ((L >> 3) & 1), lanes 16..63 repeating lanes 0..15.
 struct MetaPair {
     unsigned id, mask, base;
 };
-
-// Panel q + E (E = 0, 1) of a pair, in the per-panel lane layout: within each 16-lane DPP row the
-// half holding the other panel takes the wanted half's values (row_shr:8 into lanes 8..15 for
-// E = 0, row_shl:8 into lanes 0..7 for E = 1), one VALU move per field and no LDS round trip.
-template <unsigned E>
-__device__ __forceinline__ unsigned pairHalf(unsigned v) {
-    return E == 0 ? unsigned(__builtin_amdgcn_update_dpp(int(v), int(v), 0x118, 0xF, 0xC, false))
-                  : unsigned(__builtin_amdgcn_update_dpp(int(v), int(v), 0x108, 0xF, 0x3, false));
-}
-template <unsigned E>
-__device__ __forceinline__ Meta pairPanel(const MetaPair& m) {
-    return {pairHalf<E>(m.id), pairHalf<E>(m.mask), pairHalf<E>(m.base)};
-}
 
 // Addressing modes of the X and A-stream loads, chosen per launch on the host.
 enum : unsigned { kBuffer = 0, kGlobal = 1, kGlobalU16 = 2 };
@@ -244,14 +228,9 @@ struct Loader {
         vbase = __builtin_amdgcn_readfirstlane(m.base);
         vals = a->m.values + vbase;
     }
-    // Panel `panel`, and panels q and q + 1, clamped to `last`.
+    // Panel `panel`, clamped to `last`.
     __device__ Meta meta8(unsigned panel, unsigned last, unsigned lane) const {
         const unsigned s = (min(panel, last) - first) * 8 + (lane & 7);
-        const std::uint64_t md = __builtin_nontemporal_load(meta + s);
-        return {__builtin_nontemporal_load(ids + s), unsigned(md), unsigned(md >> 32)};
-    }
-    __device__ MetaPair meta2(unsigned q, unsigned last, unsigned lane) const {
-        const unsigned s = (min(q + ((lane >> 3) & 1u), last) - first) * 8 + (lane & 7);
         const std::uint64_t md = __builtin_nontemporal_load(meta + s);
         return {__builtin_nontemporal_load(ids + s), unsigned(md), unsigned(md >> 32)};
     }
@@ -291,13 +270,13 @@ struct RowBit {
 };
 
 // Stage 2 of one panel (exclusive: `rowBit`; shared: row groups `groups`), with the X tiles of the
-// wave's S slices; the scale too unless the caller loads it (LoadScale false).
-template <bool Shared, unsigned S, class Ld, bool LoadScale = true>
+// wave's S slices.
+template <bool Shared, unsigned S, class Ld>
 __device__ __forceinline__ void loadStage(const Ld& ld, const Meta& m, const RowBit& rowBit,
                                           unsigned groups, unsigned lane, Stage& s) {
     // Padding slots (source UINT32_MAX, metadata 0) have an empty row mask; their scale and X tile
     // read 0 (narrow) or a clamped row (wide), multiplied by A entries that are all 0.
-    if constexpr (LoadScale) s.scale = ld.scale(m.id);
+    s.scale = ld.scale(m.id);
     s.bits = 0;
     constexpr unsigned kCount = Shared ? 4 : 1;
 #pragma unroll
@@ -353,9 +332,9 @@ __device__ __forceinline__ void waveSync() {
 }
 
 struct Lds {
-    _Float16* table16; // a' (f16 path): F128 [32 rows][8 slots], F256 two areas (tableEntry)
+    _Float16* table16; // a' (f16 path), two areas (tableEntry)
     float* table32;    // [32 rows][8 slots] tf32(a) / 2 (FP32 path)
-    u32x4* xtile;      // [8 slots][blocks][128 bytes] X rows: block S * area + slice (xTile)
+    u32x4* xtile;      // X rows: xTile, or the ring of walkPairs
     float* mant;       // [2 areas][8 slots] scale mantissas of a panel
     unsigned short* redo; // [384]: offsets (from the task's first panel) of the panels that need
                           // the FP32 path, in the order found (a task has <= 384 panels)
@@ -398,37 +377,26 @@ __device__ __forceinline__ f16x8 join(f16x4 lo, f16x4 hi) {
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// A panel is computed in two parts. stagePanel writes its operands to LDS area 0 or 1: the f16 A
-// table, the X tiles and the scale mantissas. crunch reads them back, dequantizes the X blocks and
-// runs the MFMAs, over area 0 alone (one v_mfma_f32_32x32x8_f16 per 32-feature block) or over both
-// areas (one v_mfma_f32_32x32x16_f16 per block, K = the 16 slots of two panels: lane half h holds
+// A panel is computed in two parts. Its operands are written to LDS area 0 or 1 (stagePanel, or for a
+// pair at once walkPairs): the f16 A table, the X tiles and the scale mantissas. They are read back, the
+// X blocks dequantized and multiplied, over one area (one v_mfma_f32_32x32x8_f16 per 32-feature block) or
+// both (one v_mfma_f32_32x32x16_f16 per block, K = the 16 slots of two panels: lane half h holds
 // k = 8h + j, j < 4 area 0's slot 4h + j and j >= 4 area 1's slot 4h + j - 4, in both operands, so
-// each MFMA adds both panels' products). F256 computes its panels in pairs: half the MFMAs, and
-// half the matrix-core time, of one MFMA per panel and block.
+// each MFMA adds both panels' products). Pairs take half the MFMAs, and half the matrix-core time.
 //
-// Table layout: F128 (one area) [32 rows][8 slots]; F256 [32 rows][2 halves][2 areas][4 slots], so
-// that the entries of row m and slots 4h .. 4h + 3 are 8 contiguous bytes per area and 16 for both.
-// Either way they start at f16 index 4 (2m + h) * kAreas of area 0. Lane L writes slot L & 7 of row
-// 8g + (L >> 3) of row group g: F128 index 64g + L.
-template <unsigned S>
+// Table layout: [32 rows][2 halves][2 areas][4 slots], so that the entries of row m and slots
+// 4h .. 4h + 3 are 8 contiguous bytes per area and 16 for both, from f16 index 8 (2m + h) on. Here: the
+// entry of slot L & 7 of row 8g + (L >> 3) of row group g.
 __device__ __forceinline__ unsigned tableEntry(unsigned g, unsigned lane, unsigned area) {
-    if constexpr (S == 1) {
-        return 64 * g + lane;
-    } else {
-        const unsigned row = 8 * g + (lane >> 3), slot = lane & 7;
-        return ((row * 2 + (slot >> 2)) * 2 + area) * 4 + (slot & 3);
-    }
+    const unsigned row = 8 * g + (lane >> 3), slot = lane & 7;
+    return ((row * 2 + (slot >> 2)) * 2 + area) * 4 + (slot & 3);
 }
 
-// X tiles in LDS: [8 slots][blocks][128 bytes], block S * area + slice (F128: one block; F256: four,
-// two areas of two slices). Returns the 16-byte index of the first tile of (slot, block). A lane
-// reads dword m of slots 4h .. 4h + 3 of every block: at F256 its 16 reads of a pair lie within 2 KB
-// of its first one, so two base addresses 1 KB apart reach them all through the 8-bit dword offsets
-// of two-address LDS reads (with one block per 1 KB, as [block][slot], it took four).
+// X tiles in LDS of walkPanels and the FP32 pass: [8 slots][2 S blocks][128 bytes], block S * area +
+// slice. Returns the 16-byte index of the first tile of (slot, block).
 template <unsigned S>
 __device__ __forceinline__ unsigned xTile(unsigned slot, unsigned block) {
-    constexpr unsigned kBlocks = S == 1 ? 1 : 2 * S;
-    return (slot * kBlocks + block) * 8;
+    return (slot * 2 * S + block) * 8;
 }
 
 // Writes panel `s` to LDS area `area`. Per lane: slot lane & 7, row lane >> 3 of each row group; an
@@ -464,7 +432,7 @@ __device__ __forceinline__ bool stagePanel(const Stage& s, unsigned lane, const 
     const bool useF16 = inexact == 0;
 #pragma unroll
     for (unsigned j = 0; j < kCount; ++j)
-        lds.table16[Shared ? tableEntry<S>(j, lane, area) : entry] =
+        lds.table16[Shared ? tableEntry(j, lane, area) : entry] =
             useF16 ? ap[j] : static_cast<_Float16>(0.0f);
 #pragma unroll
     for (unsigned k = 0; k < S; ++k) lds.xtile[xTile<S>(lane >> 3, S * area + k) + (lane & 7)] = s.x[k];
@@ -484,85 +452,73 @@ __device__ __forceinline__ f16x4 dequantBlock(const unsigned (&d)[4], const f32x
         f16x4, __builtin_shufflevector(roundPack(q[0], q[1]), roundPack(q[2], q[3]), 0, 1, 2, 3));
 }
 
-// The MFMAs of area 0 (Pair false) or of areas 0 and 1 (Pair true). The S x 4 blocks are
-// dequantized one ahead of their MFMAs: block i + 1's conversions run between block i's last pack
-// and its MFMA, so the MFMA's operand was written a dozen VALU instructions before it is read and
-// needs no wait states.
-template <unsigned S, bool Pair>
-__device__ __forceinline__ void crunch(const Lds& lds, f32x16 (&acc)[4 * S], LaneMh mh) {
-    constexpr unsigned kAreas = Pair ? 2 : 1;
-    waveSync();
-    const unsigned m = mh.m, h = mh.h;
-    f32x4 mant[kAreas];
-    unsigned d[kAreas][S][4];
-#pragma unroll
-    for (unsigned r = 0; r < kAreas; ++r) {
-        mant[r] = reinterpret_cast<const f32x4*>(lds.mant + 8 * r)[h];
-#pragma unroll
-        for (unsigned k = 0; k < S; ++k) {
-            const unsigned* xw = reinterpret_cast<const unsigned*>(lds.xtile) + m;
-#pragma unroll
-            for (unsigned i = 0; i < 4; ++i) d[r][k][i] = xw[4 * xTile<S>(4 * h + i, S * r + k)];
-        }
-    }
+// A lane's operands of one panel (Areas == 1) or of a pair of panels (2), read back from LDS: the X dwords
+// of its four slots, their mantissas, and its row's A entries.
+template <unsigned S, unsigned Areas>
+struct Operands {
+    unsigned d[Areas][S][4];
+    f32x4 mant[Areas];
+    std::conditional_t<Areas == 1, f16x4, f16x8> b;
+};
+
+// The MFMAs of one panel or of a pair. The S x 4 blocks are dequantized one ahead of their MFMAs: block
+// i + 1's conversions run between block i's last pack and its MFMA, so the MFMA's operand was written
+// a dozen VALU instructions before it is read and needs no wait states.
+template <unsigned S, unsigned Areas>
+__device__ __forceinline__ void multiply(const Operands<S, Areas>& o, f32x16 (&acc)[4 * S]) {
     using I0 = std::integral_constant<unsigned, 0>;
     using I1 = std::integral_constant<unsigned, 1>;
     using I2 = std::integral_constant<unsigned, 2>;
     using I3 = std::integral_constant<unsigned, 3>;
-    if constexpr (Pair) {
-        const f16x8 b = reinterpret_cast<const f16x8*>(lds.table16)[m * 2 + h];
-        auto op = [&](auto blk, unsigned k) {
-            constexpr unsigned B = decltype(blk)::value;
-            return join(dequantBlock<B>(d[0][k], mant[0]), dequantBlock<B>(d[1][k], mant[1]));
-        };
-        auto mfma = [&](unsigned t, f16x8 x) {
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, b, acc[t], 0, 0, 0);
-        };
-        f16x8 av = op(I0{}, 0);
+    auto op = [&](auto blk, unsigned k) {
+        constexpr unsigned B = decltype(blk)::value;
+        if constexpr (Areas == 2)
+            return join(dequantBlock<B>(o.d[0][k], o.mant[0]), dequantBlock<B>(o.d[1][k], o.mant[1]));
+        else
+            return dequantBlock<B>(o.d[0][k], o.mant[0]);
+    };
+    auto mfma = [&](unsigned t, auto x) {
+        if constexpr (Areas == 2)
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, o.b, acc[t], 0, 0, 0);
+        else
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x8f16(x, o.b, acc[t], 0, 0, 0);
+    };
+    auto av = op(I0{}, 0);
 #pragma unroll
-        for (unsigned k = 0; k < S; ++k) {
-            f16x8 nx = op(I1{}, k);
-            mfma(4 * k + 0, av);
-            av = op(I2{}, k);
-            mfma(4 * k + 1, nx);
-            nx = op(I3{}, k);
-            mfma(4 * k + 2, av);
-            if (k + 1 < S) av = op(I0{}, k + 1);
-            mfma(4 * k + 3, nx);
-        }
-    } else {
-        const f16x4 b = reinterpret_cast<const f16x4*>(lds.table16)[(m * 2 + h) * (S == 1 ? 1 : 2)];
-        auto op = [&](auto blk, unsigned k) {
-            constexpr unsigned B = decltype(blk)::value;
-            return dequantBlock<B>(d[0][k], mant[0]);
-        };
-        auto mfma = [&](unsigned t, f16x4 x) {
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x8f16(x, b, acc[t], 0, 0, 0);
-        };
-        f16x4 av = op(I0{}, 0);
-#pragma unroll
-        for (unsigned k = 0; k < S; ++k) {
-            f16x4 nx = op(I1{}, k);
-            mfma(4 * k + 0, av);
-            av = op(I2{}, k);
-            mfma(4 * k + 1, nx);
-            nx = op(I3{}, k);
-            mfma(4 * k + 2, av);
-            if (k + 1 < S) av = op(I0{}, k + 1);
-            mfma(4 * k + 3, nx);
-        }
+    for (unsigned k = 0; k < S; ++k) {
+        auto nx = op(I1{}, k);
+        mfma(4 * k + 0, av);
+        av = op(I2{}, k);
+        mfma(4 * k + 1, nx);
+        nx = op(I3{}, k);
+        mfma(4 * k + 2, av);
+        if (k + 1 < S) av = op(I0{}, k + 1);
+        mfma(4 * k + 3, nx);
     }
-    waveSync();
 }
 
-// One panel alone: staged in area 0 and computed.
-template <bool Wide, bool Shared, unsigned S>
-__device__ __forceinline__ bool computePanelF16(const Stage& s, unsigned lane, const Lds& lds,
-                                                f32x16 (&acc)[4 * S], unsigned entry, unsigned keep,
-                                                LaneMh mh) {
-    const bool useF16 = stagePanel<Wide, Shared, S>(s, lane, lds, 0, entry, keep);
-    crunch<S, false>(lds, acc, mh);
-    return useF16;
+// Reads the operands of area First, or of both areas (Areas == 2), and multiplies.
+template <unsigned S, unsigned Areas, unsigned First = 0>
+__device__ __forceinline__ void crunch(const Lds& lds, f32x16 (&acc)[4 * S], LaneMh mh) {
+    waveSync();
+    const unsigned m = mh.m, h = mh.h;
+    Operands<S, Areas> o;
+#pragma unroll
+    for (unsigned r = 0; r < Areas; ++r) {
+        o.mant[r] = reinterpret_cast<const f32x4*>(lds.mant + 8 * (First + r))[h];
+#pragma unroll
+        for (unsigned k = 0; k < S; ++k) {
+            const unsigned* xw = reinterpret_cast<const unsigned*>(lds.xtile) + m;
+#pragma unroll
+            for (unsigned i = 0; i < 4; ++i) o.d[r][k][i] = xw[4 * xTile<S>(4 * h + i, S * (First + r) + k)];
+        }
+    }
+    if constexpr (Areas == 2)
+        o.b = reinterpret_cast<const f16x8*>(lds.table16)[m * 2 + h];
+    else
+        o.b = reinterpret_cast<const f16x4*>(lds.table16)[(m * 2 + h) * 2 + First];
+    multiply<S, Areas>(o, acc);
+    waveSync();
 }
 
 // A shared-kind panel with exact FP32 operands (v_mfma_f32_32x32x2_f32): K = 2 steps over slot
@@ -649,6 +605,10 @@ struct GroupBounds {
     __device__ unsigned end(unsigned g) const {
         return g == 0 ? b0 : g == 1 ? b1 : g == 2 ? b2 : 0xFFFFFFFFu;
     }
+    // Row group of panel p (the ends do not decrease).
+    __device__ unsigned of(unsigned p) const {
+        return unsigned(p >= b0) + unsigned(p >= b1) + unsigned(p >= b2);
+    }
 };
 
 // Row group of the exclusive panels of one task, walked in increasing panel order. Wave-uniform, in
@@ -656,44 +616,29 @@ struct GroupBounds {
 struct GroupCursor {
     unsigned g, end;
     __device__ void advance(const GroupBounds& b, unsigned p) {
-        while (p >= end) end = b.end(++g);
+        g = b.of(p);
+        end = b.end(g);
     }
 };
 
-// The panels [lo, hi) of one kind, pipelined, two panels per iteration with the odd one after the
-// loop (a single exit keeps the accumulators in place). The loads run past the end of the walk: they
-// read the next bucket's panels, nothing or the last panel again (Loader), and are never computed.
-// `first` is panel lo's metadata, loaded by the caller if
-// lo is the task's first panel (beside the bucket bounds, one dependent load earlier).
-//
-// The four exclusive buckets are one walk: the loads run ahead across a bucket's end, and only the
-// row bit of the loads and the table entry of the writes change there (wave-uniform branches, taken
-// at most three times a task). One loop per bucket instead emptied the pipeline four times per task,
-// about 2 us of cold loads each.
-//
-// F128 (S == 1) loads the metadata, sourceIds and scales of two panels with one instruction each, one
-// iteration ahead, and hands each panel its slots by DPP row shifts: per panel that is one and
-// a half vector memory instructions fewer (c3: 3.51 -> 3.39 ms). F256, at two waves per SIMD, keeps
-// one metadata load per panel (pairs cost it 0.5-2% in every form tried) and keeps two panels of
-// gathers in flight: stage data two panels ahead, metadata four (1.2% faster than one panel ahead;
-// three ahead gained 0.2% for 16 more registers), and computes its panels in pairs, K = 16 per MFMA
-// (c3: 5.92 -> 5.72 ms).
+// The panels [lo, hi) of the 64-bit-addressed instances, all exclusive or of any kind (Shared), in the
+// pairs and with the products of walkPairs, one panel's loads and table entries at a time. `first` is
+// panel lo's metadata if lo is the wave's first panel (loaded by the caller beside the bucket bounds, one
+// dependent load earlier). Stage data two panels ahead, metadata four: three stage buffers rotate, at the
+// step of panel i holding panels i, i + 1 and (loaded there) i + 2. Loads past the end repeat the last
+// panel and are never computed.
 template <bool Shared, unsigned S, class Ld>
 __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBounds& bounds,
                                            unsigned lo, unsigned hi, Meta first,
                                            f32x16 (&acc)[4 * S]) {
     if (lo >= hi) return;
-    constexpr unsigned kAreas = S == 1 ? 1 : 2;
-    const unsigned n = hi - lo, lane = w.lane;
-    const unsigned last = hi - 1;
-    const unsigned pairs = n / 2;
+    const unsigned n = hi - lo, lane = w.lane, last = w.end - 1;
     // The loads' side of a bucket change: to be called before the loads of panel p, for increasing p.
     // Returns a shared panel's row groups.
-    BucketCursor bucket{w.offsets, 5, Shared ? w.offsets[6] : 0u};
-    GroupCursor loads{0, bounds.b0};
-    loads.advance(bounds, lo);
+    BucketCursor bucket{w.offsets, 1, Shared ? w.offsets[2] : 0u};
+    GroupCursor loads{0, 0};
     const unsigned bit0 = 1u << (lane >> 3);
-    RowBit rowBit{bit0 << (8 * loads.g), (bit0 << (8 * loads.g)) - 1u};
+    RowBit rowBit{};
     auto enter = [&](unsigned p) __attribute__((always_inline)) {
         if constexpr (Shared) return bucket.groups(min(p, last));
         if (__builtin_expect(p >= loads.end, 0)) {
@@ -704,118 +649,391 @@ __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBound
         return 0u;
     };
     // The table's side: an area's table holds one row group at a time, the other groups' entries 0.
-    GroupCursor staged[kAreas];
-    unsigned entry[kAreas];
-#pragma unroll
-    for (unsigned a = 0; a < kAreas; ++a) {
-        staged[a] = loads;
-        entry[a] = tableEntry<S>(loads.g, lane, a);
-    }
+    GroupCursor staged[2] = {{0, 0}, {0, 0}};
+    unsigned entry[2] = {tableEntry(0, lane, 0), tableEntry(0, lane, 1)};
     if constexpr (!Shared) {
 #pragma unroll
-        for (unsigned i = 0; i < 2 * kAreas; ++i)
+        for (unsigned i = 0; i < 4; ++i)
             reinterpret_cast<f16x2*>(w.lds.table16)[64 * i + lane] = f16x2{0, 0};
     }
-    auto enterTable = [&](unsigned p, unsigned a) __attribute__((always_inline)) {
+    auto stage = [&](const Stage& st, unsigned p, auto area) __attribute__((always_inline)) {
+        constexpr unsigned A = decltype(area)::value;
         if constexpr (!Shared) {
-            if (__builtin_expect(p >= staged[a].end, 0)) {
-                w.lds.table16[entry[a]] = static_cast<_Float16>(0.0f);
-                staged[a].advance(bounds, p);
-                entry[a] = tableEntry<S>(staged[a].g, lane, a);
+            if (__builtin_expect(p >= staged[A].end, 0)) {
+                w.lds.table16[entry[A]] = static_cast<_Float16>(0.0f);
+                staged[A].advance(bounds, p);
+                entry[A] = tableEntry(staged[A].g, lane, A);
             }
         }
+        flagRedo(w, p, !stagePanel<Ld::kWide, Shared, S>(st, lane, w.lds, A, entry[A], w.keep));
     };
-    // Panel p alone, in area 0.
-    auto computeOne = [&](const Stage& st, unsigned p) __attribute__((always_inline)) {
-        enterTable(p, 0);
-        flagRedo(w, p, !computePanelF16<Ld::kWide, Shared, S>(st, lane, w.lds, acc, entry[0], w.keep, w.mh));
+    auto computePair = [&]() __attribute__((always_inline)) {
+        if constexpr (Shared && S == 1) { // as walkPairs
+            crunch<S, 1, 0>(w.lds, acc, w.mh);
+            crunch<S, 1, 1>(w.lds, acc, w.mh);
+        } else {
+            crunch<S, 2>(w.lds, acc, w.mh);
+        }
     };
-    Stage sa, sb;
+    using Area0 = std::integral_constant<unsigned, 0>;
+    using Area1 = std::integral_constant<unsigned, 1>;
     if (lo != w.begin) first = ld.meta8(lo, lo, lane);
-    if constexpr (S == 1) {
-        MetaPair pair = ld.meta2(lo + 1, last, lane); // panels lo + 1, lo + 2
-        __builtin_amdgcn_sched_barrier(0);
-        if (lo == w.begin) ld.startTask(first);
-        loadStage<Shared, S>(ld, first, rowBit, enter(lo), lane, sa);
-        // Each panel's row shifts run half an iteration before its loads need them.
-        Meta mFirst = pairPanel<0>(pair);
-#pragma unroll 1
-        for (unsigned k = 0; k < pairs; ++k) {
-            // Computes panels lo + 2k (in sa) and lo + 2k + 1; loads the pair after next.
-            const unsigned gb = enter(lo + 2 * k + 1);
-            const MetaPair next = ld.meta2(lo + 2 * k + 3, last, lane);
-            const float sc = ld.scale(pair.id); // both panels' scales, laid out as `pair`
-            loadStage<Shared, S, Ld, false>(ld, mFirst, rowBit, gb, lane, sb);
-            const Meta mSecond = pairPanel<1>(pair);
-            // Issue this half's loads before any use of the previous half's: the vmcnt counter
-            // is in order, so computing first would wait for loads issued only half an
-            // iteration ago.
-            __builtin_amdgcn_sched_barrier(0);
-            computeOne(sa, lo + 2 * k);
-            const unsigned ga = enter(lo + 2 * k + 2);
-            loadStage<Shared, S, Ld, false>(ld, mSecond, rowBit, ga, lane, sa);
-            __builtin_amdgcn_sched_barrier(0);
-            sb.scale = __uint_as_float(pairHalf<0>(__float_as_uint(sc)));
-            computeOne(sb, lo + 2 * k + 1);
-            sa.scale = __uint_as_float(pairHalf<1>(__float_as_uint(sc)));
-            pair = next;
-            mFirst = pairPanel<0>(pair);
-        }
-        if (n & 1) computeOne(sa, last);
-    } else {
-        // F256: stage data two panels ahead, metadata four. Three stage buffers rotate: at the step
-        // of panel i they hold panels i, i + 1 and (loaded there) i + 2.
-        Stage sc;
-        const Meta second = ld.meta8(lo + 1, last, lane);
-        // The steps expect m1's loads to be older than m2's (waits are counted in issue order).
-        Meta m1 = ld.meta8(lo + 2, last, lane);
-        __builtin_amdgcn_sched_barrier(0);
-        Meta m2 = ld.meta8(lo + 3, last, lane);
-        __builtin_amdgcn_sched_barrier(0);
-        if (lo == w.begin) ld.startTask(first);
-        loadStage<Shared, S>(ld, first, rowBit, enter(lo), lane, sa);
-        loadStage<Shared, S>(ld, second, rowBit, enter(lo + 1), lane, sb);
-        // Step of panel `panel` (in `cur`): the loads of panel + 2 into `ahead`, then the panel staged
-        // in area 0 (first of a pair) or staged in area 1 and the pair computed (second).
-        auto step = [&](auto second, Stage& cur, Stage& ahead,
-                        unsigned panel) __attribute__((always_inline)) {
-            loadStage<Shared, S>(ld, m1, rowBit, enter(panel + 2), lane, ahead);
-            m1 = m2;
-            m2 = ld.meta8(panel + 4, last, lane);
-            __builtin_amdgcn_sched_barrier(0);
-            constexpr bool kSecond = decltype(second)::value;
-            constexpr unsigned kArea = kSecond ? 1u : 0u;
-            enterTable(panel, kArea);
-            flagRedo(w, panel, !stagePanel<Ld::kWide, Shared, S>(cur, lane, w.lds, kArea, entry[kArea], w.keep));
-            if constexpr (kSecond) crunch<S, true>(w.lds, acc, w.mh);
-        };
-        using First = std::integral_constant<bool, false>;
-        using Second = std::integral_constant<bool, true>;
-        // Panels in pairs, in a loop unrolled by six (the period of both the pairs and the stage
-        // rotation), then the r < 6 panels left: their pairs by the same steps and a last panel
-        // without a partner alone, staged in area 0. (A loop that leaves after any panel, computing
-        // the unpaired one on its way out, made the register allocator spill the accumulators.)
-        const unsigned sixes = n / 6, r = n - 6 * sixes;
-        unsigned i = lo;
-#pragma unroll 1
-        for (unsigned k = 0; k < sixes; ++k, i += 6) {
-            step(First{}, sa, sc, i);
-            step(Second{}, sb, sa, i + 1);
-            step(First{}, sc, sb, i + 2);
-            step(Second{}, sa, sc, i + 3);
-            step(First{}, sb, sa, i + 4);
-            step(Second{}, sc, sb, i + 5);
-        }
-        if (r >= 2) {
-            step(First{}, sa, sc, i);
-            step(Second{}, sb, sa, i + 1);
-        }
-        if (r >= 4) {
-            step(First{}, sc, sb, i + 2);
-            step(Second{}, sa, sc, i + 3);
-        }
-        if (r & 1) computeOne(r == 1 ? sa : r == 3 ? sc : sb, hi - 1);
+    const Meta next = ld.meta8(lo + 1, last, lane);
+    // The steps expect m1's loads to be older than m2's (waits are counted in issue order).
+    Meta m1 = ld.meta8(lo + 2, last, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    Meta m2 = ld.meta8(lo + 3, last, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    if (lo == w.begin) ld.startTask(first);
+    Stage sa, sb, sc;
+    {
+        const unsigned g0 = enter(lo);
+        loadStage<Shared, S>(ld, first, rowBit, g0, lane, sa);
+        const unsigned g1 = enter(lo + 1);
+        loadStage<Shared, S>(ld, next, rowBit, g1, lane, sb);
     }
+    auto step = [&](auto area, Stage& cur, Stage& ahead, unsigned panel) __attribute__((always_inline)) {
+        const unsigned g = enter(panel + 2);
+        loadStage<Shared, S>(ld, m1, rowBit, g, lane, ahead);
+        m1 = m2;
+        m2 = ld.meta8(panel + 4, last, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        stage(cur, panel, area);
+        if constexpr (decltype(area)::value == 1) computePair();
+    };
+    // Panels in pairs, in a loop unrolled by six (the period of both the pairs and the stage rotation),
+    // then the r < 6 panels left: their pairs by the same steps and a last panel with an empty one.
+    const unsigned sixes = n / 6, r = n - 6 * sixes;
+    unsigned i = lo;
+#pragma unroll 1
+    for (unsigned k = 0; k < sixes; ++k, i += 6) {
+        step(Area0{}, sa, sc, i);
+        step(Area1{}, sb, sa, i + 1);
+        step(Area0{}, sc, sb, i + 2);
+        step(Area1{}, sa, sc, i + 3);
+        step(Area0{}, sb, sa, i + 4);
+        step(Area1{}, sc, sb, i + 5);
+    }
+    if (r >= 2) {
+        step(Area0{}, sa, sc, i);
+        step(Area1{}, sb, sa, i + 1);
+    }
+    if (r >= 4) {
+        step(Area0{}, sc, sb, i + 2);
+        step(Area1{}, sa, sc, i + 3);
+    }
+    if (r & 1) {
+        const Stage odd = r == 1 ? sa : r == 3 ? sc : sb;
+        stage(odd, hi - 1, Area0{});
+        stagePanel<Ld::kWide, Shared, S>(Stage{}, lane, w.lds, 1, entry[1], w.keep);
+        computePair();
+    }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Panel walk of the buffer-addressed instances: two panels at a time, with the same products as
+// walkPanels.
+//
+// Bound by VALU issue wherever the gathers do not run at the memory system's request rate, so the
+// instructions per panel decide. A pair's 16 slots fill a 16-lane row: lane L holds slot L & 7 of
+// panel (L >> 3) & 1 in its metadata, scale, A values (rows (L >> 4) + 4j of the row group, j = 0, 1)
+// and table entries, so nothing is moved between lanes to separate the panels; the scale's work is done
+// once per pair; and the pair is one v_mfma_f32_32x32x16_f16 per 32-feature block. X goes straight from
+// memory to LDS (16 bytes per lane), so rows in flight take no registers and F128's pairs fit its 128.
+// Against one panel at a time at F128 and pairs staged panel by panel at F256, X through registers (us):
+// 100K rows F128 74.5 -> 65.2, 262K power law F128 221 -> 213, F256 361 -> 355, 2.45M rows F128
+// 2,872 -> 2,802, F256 4,884 -> 4,761. Loads to LDS alone, with the rest as before, gained nothing
+// (F128 +0.1 to +4%): the depth of the gathers is not what bounds them.
+//
+// LDS of a wave: a ring of two pairs' X rows, [panel & 3][slice][8 slots][128 bytes] as the loads deliver
+// them (lane L: 16 bytes at 16 L); the A table [32 rows][2 halves][2 panels][4 slots]; the mantissas
+// [2 panels][8 slots].
+//
+// The compiler orders every LDS access it knows of after the last load to LDS, which would empty the
+// pipeline at each pair. So the accesses of the loop (table entries, mantissas and operands) are written
+// out below, and the wait in front of the operand reads is counted by hand: the loop issues its vector
+// memory instructions in a fixed order (the scheduling barriers keep it), a pair's X last, and kYounger
+// of them, the next pair's, follow before it is read. Only added memory instructions, that is spills,
+// could make the count too high, and the build refuses those.
+
+__device__ __forceinline__ unsigned ldsAddress(const void* p) {
+    return unsigned(reinterpret_cast<std::uintptr_t>(
+        (const __attribute__((address_space(3))) void*)p));
+}
+
+// Row groups of the pairs of an exclusive walk, in scalar registers: a pair inside one bucket costs a
+// compare and an untaken branch.
+struct PairCursor {
+    unsigned g = 0, second = 0; // row groups of the pair's panels
+    unsigned limit = 0;         // pairs whose second panel lies before it need no update
+    __device__ bool changes(unsigned p) const { return __builtin_expect(p + 1 >= limit, 0); }
+    __device__ void update(const GroupBounds& b, unsigned p) {
+        g = b.of(p);
+        second = b.of(p + 1);
+        limit = second == g ? b.end(g) : 0u;
+    }
+};
+
+// The lane's LDS byte addresses: its X dwords in ring slot 0, and its mantissas.
+struct LaneLds {
+    unsigned x, tableRead, mantWrite, mantRead;
+};
+
+// Waits until at most Younger vector memory instructions are outstanding, then reads a pair's operands
+// (X from LDS address x).
+template <unsigned S, unsigned Younger>
+__device__ __forceinline__ void readPair(Operands<S, 2>& o, const LaneLds& at, unsigned x) {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    auto put = [&](unsigned r, unsigned k, u32x2 lo, u32x2 hi) {
+        o.d[r][k][0] = lo[0];
+        o.d[r][k][1] = lo[1];
+        o.d[r][k][2] = hi[0];
+        o.d[r][k][3] = hi[1];
+    };
+    u32x2 a, b;
+    if constexpr (S == 1) { // one address: the second panel's rows lie past the reach of two-address reads
+        asm volatile("s_waitcnt vmcnt(%12)\n\t"
+                     "ds_read2_b32 %0, %9 offset1:32\n\t"
+                     "ds_read2_b32 %1, %9 offset0:64 offset1:96\n\t"
+                     "ds_read_b32 %2, %9 offset:1024\n\t"
+                     "ds_read_b32 %3, %9 offset:1152\n\t"
+                     "ds_read_b32 %4, %9 offset:1280\n\t"
+                     "ds_read_b32 %5, %9 offset:1408\n\t"
+                     "ds_read_b128 %6, %10\n\t"
+                     "ds_read_b128 %7, %10 offset:32\n\t"
+                     "ds_read_b128 %8, %11\n\t"
+                     "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(a), "=&v"(b), "=&v"(o.d[1][0][0]), "=&v"(o.d[1][0][1]),
+                       "=&v"(o.d[1][0][2]), "=&v"(o.d[1][0][3]), "=&v"(o.mant[0]),
+                       "=&v"(o.mant[1]), "=&v"(o.b)
+                     : "v"(x), "v"(at.mantRead), "v"(at.tableRead), "n"(Younger)
+                     : "memory");
+        put(0, 0, a, b);
+    } else {
+        u32x2 c, d, e, f, g, h;
+        const unsigned x0b = x + 1024, x1 = x + 2048, x1b = x + 3072;
+        asm volatile("s_waitcnt vmcnt(%17)\n\t"
+                     "ds_read2_b32 %0, %11 offset1:32\n\t"
+                     "ds_read2_b32 %1, %11 offset0:64 offset1:96\n\t"
+                     "ds_read2_b32 %2, %13 offset1:32\n\t"
+                     "ds_read2_b32 %3, %13 offset0:64 offset1:96\n\t"
+                     "ds_read_b128 %8, %15\n\t"
+                     "ds_read_b128 %9, %15 offset:32\n\t"
+                     "ds_read_b128 %10, %16\n\t"
+                     "ds_read2_b32 %4, %12 offset1:32\n\t"
+                     "ds_read2_b32 %5, %12 offset0:64 offset1:96\n\t"
+                     "ds_read2_b32 %6, %14 offset1:32\n\t"
+                     "ds_read2_b32 %7, %14 offset0:64 offset1:96\n\t"
+                     "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(a), "=&v"(b), "=&v"(c), "=&v"(d), "=&v"(e), "=&v"(f), "=&v"(g), "=&v"(h),
+                       "=&v"(o.mant[0]), "=&v"(o.mant[1]), "=&v"(o.b)
+                     : "v"(x), "v"(x0b), "v"(x1), "v"(x1b), "v"(at.mantRead), "v"(at.tableRead),
+                       "n"(Younger)
+                     : "memory");
+        put(0, 0, a, b);
+        put(1, 0, c, d);
+        put(0, 1, e, f);
+        put(1, 1, g, h);
+    }
+}
+
+// The same for panel A of a pair alone, at F128.
+template <unsigned A, unsigned Younger>
+__device__ __forceinline__ void readPanel(Operands<1, 1>& o, const LaneLds& at, unsigned x) {
+    asm volatile("s_waitcnt vmcnt(%9)\n\t"
+                 "ds_read_b32 %0, %6 offset:%10\n\t"
+                 "ds_read_b32 %1, %6 offset:%10+128\n\t"
+                 "ds_read_b32 %2, %6 offset:%10+256\n\t"
+                 "ds_read_b32 %3, %6 offset:%10+384\n\t"
+                 "ds_read_b128 %4, %7 offset:%11\n\t"
+                 "ds_read_b64 %5, %8 offset:%12\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(o.d[0][0][0]), "=&v"(o.d[0][0][1]), "=&v"(o.d[0][0][2]), "=&v"(o.d[0][0][3]),
+                   "=&v"(o.mant[0]), "=&v"(o.b)
+                 : "v"(x), "v"(at.mantRead), "v"(at.tableRead), "n"(Younger), "n"(1024 * A),
+                   "n"(32 * A), "n"(8 * A)
+                 : "memory");
+}
+
+// Table entry offsets in bytes: pass j (rows + 4j) and row group g of a lane's entry.
+constexpr unsigned kPassBytes = 128, kGroupBytes = 256;
+
+__device__ __forceinline__ void writeEntry(unsigned address, unsigned offset, _Float16 v) {
+    asm volatile("ds_write_b16 %0, %1 offset:%2" ::"v"(address), "v"(v), "n"(offset) : "memory");
+}
+
+// Issues a pair's X rows, to ring slots 2 (k & 1) and 2 (k & 1) + 1.
+template <unsigned S>
+__device__ __forceinline__ void gatherPair(const Loader<kBuffer>& ld, const TaskWalk& w, unsigned id,
+                                           unsigned k) {
+    unsigned row[2];
+#pragma unroll
+    for (unsigned a = 0; a < 2; ++a)
+        row[a] = (lanePermute(id, (w.lane >> 3) + 8 * a) << ld.xShift) + 16 * (w.lane & 7);
+    char* slot = reinterpret_cast<char*>(w.lds.xtile) + (k & 1u) * 2 * S * 1024;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (unsigned a = 0; a < 2; ++a)
+#pragma unroll
+        for (unsigned s = 0; s < S; ++s)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                ld.x, (__attribute__((address_space(3))) void*)(slot + 1024 * (S * a + s)), 16, row[a],
+                kSlice * s, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+template <unsigned Offset>
+__device__ __forceinline__ void clearWord(unsigned address) {
+    asm volatile("ds_write_b32 %0, %1 offset:%2" ::"v"(address), "v"(0u), "n"(Offset) : "memory");
+}
+
+// What one pair's step leaves for the next: the next pair's scales (lane L: slot L & 7 of panel
+// (L >> 3) & 1) and the metadata of the pair after it. The next pair's X is on its way.
+struct PairPipe {
+    MetaPair ahead;
+    float scale;
+};
+
+// The pairs [k0, k1) of a wave's panels [begin, end), all exclusive or of any kind (Shared). `cur` is
+// the metadata of pair k0; pairs after `lastPair` are never computed and load nothing of X.
+template <bool Shared, unsigned S>
+__device__ __forceinline__ void walkPairs(Loader<kBuffer>& ld, TaskWalk& w, const GroupBounds& bounds,
+                                          unsigned k0, unsigned k1, unsigned lastPair,
+                                          const MetaPair& cur, PairPipe& pipe, f32x16 (&acc)[4 * S]) {
+    constexpr unsigned kValues = Shared ? 8 : 2; // A values of a lane per pair: [row group][pass]
+    const unsigned lane = w.lane, last = w.end - 1;
+    const bool second = (lane & 8) != 0; // the lane's panel of a pair
+    const unsigned bit0 = 1u << (lane >> 4);
+    const unsigned table = ldsAddress(w.lds.table16) +
+                           2 * (((lane >> 4) * 2 + ((lane & 7) >> 2)) * 8 + (second ? 4 : 0) + (lane & 3));
+    const LaneLds at{ldsAddress(w.lds.xtile) + 4 * w.mh.m + 512 * w.mh.h,
+                     ldsAddress(w.lds.table16) + 16 * (2 * w.mh.m + w.mh.h),
+                     ldsAddress(w.lds.mant) + 4 * (lane & 15), ldsAddress(w.lds.mant) + 16 * w.mh.h};
+
+    // A pair's A values. Exclusive: `bits` is the lane's row bit of pass 0.
+    PairCursor loads;
+    BucketCursor bucket{w.offsets, 1, Shared ? w.offsets[2] : 0u};
+    unsigned bits = 0;
+    auto loadValues = [&](const MetaPair& m, unsigned p, float (&v)[kValues]) __attribute__((always_inline)) {
+        unsigned present = m.mask;
+        if constexpr (Shared) {
+            // Only the row groups of the panel's bucket.
+            auto bytes = [](unsigned g) {
+                return (g & 1u) * 0xFFu | (g & 2u) * 0x7F80u | (g & 4u) * 0x3FC000u | (g & 8u) * 0x1FE00000u;
+            };
+            const unsigned g0 = bytes(bucket.groups(min(p, last)));
+            const unsigned g1 = bytes(bucket.groups(min(p + 1, last)));
+            present &= second ? g1 : g0;
+        } else if (loads.changes(p)) {
+            loads.update(bounds, p);
+            const unsigned g0 = loads.g, g1 = loads.second;
+            bits = bit0 << (8 * (second ? g1 : g0));
+        }
+#pragma unroll
+        for (unsigned j = 0; j < kValues; ++j) {
+            const unsigned bit = Shared ? bit0 << (4 * j) : bits << (4 * j);
+            v[j] = ld.value(m.base + __popc(m.mask & (bit - 1u)), (present & bit) != 0);
+        }
+    };
+    constexpr unsigned kYounger = 3 + kValues + 2 * S; // metadata (2), scales, values, X
+
+    // The table holds one row group per panel, the other groups' entries 0.
+    PairCursor staged;
+    unsigned entry = table;
+    if constexpr (!Shared) {
+        const unsigned words = ldsAddress(w.lds.table16) + 4 * lane;
+        clearWord<0>(words);
+        clearWord<256>(words);
+        clearWord<512>(words);
+        clearWord<768>(words);
+    }
+    auto stage = [&](const float (&v)[kValues], float scale, unsigned p) __attribute__((always_inline)) {
+        if (!Shared && staged.changes(p)) {
+            writeEntry(entry, 0, 0);
+            writeEntry(entry, kPassBytes, 0);
+            staged.update(bounds, p);
+            const unsigned g0 = staged.g, g1 = staged.second;
+            entry = table + kGroupBytes * (second ? g1 : g0);
+        }
+        // stagePanel explains the scale factor and the exactness check.
+        const float pow2 = __builtin_amdgcn_ldexpf(
+            __uint_as_float(__float_as_uint(scale) & 0x7F800000u), kShift + 1);
+        std::uint64_t inexact = 0;
+        forEachIndex<kValues>([&](auto c) __attribute__((always_inline)) {
+            constexpr unsigned j = decltype(c)::value;
+            const float a = roundTf32(v[j]);
+            const _Float16 e = static_cast<_Float16>(a * pow2);
+            inexact |= __builtin_amdgcn_ballot_w64(a != 0.0f) & ~normalF16(e);
+            writeEntry(entry, kPassBytes * j, e);
+        });
+        asm volatile("ds_write_b32 %0, %1" ::"v"(at.mantWrite), "v"(shiftedMantissa(scale, w.keep))
+                     : "memory");
+        if (__builtin_expect(inexact != 0, 0)) { // the FP32 pass adds these panels: all-zero tables here
+            constexpr std::uint64_t kFirst = 0x00FF00FF00FF00FFull;
+            const bool bad0 = (inexact & kFirst) != 0, bad1 = (inexact & ~kFirst) != 0;
+            if (second ? bad1 : bad0)
+                forEachIndex<kValues>([&](auto c) __attribute__((always_inline)) {
+                    writeEntry(entry, kPassBytes * decltype(c)::value, 0);
+                });
+            flagRedo(w, p, bad0);
+            flagRedo(w, p + 1, bad1);
+        }
+    };
+
+    float v[kValues];
+    loadValues(cur, w.begin + 2 * k0, v);
+#pragma unroll 1
+    for (unsigned k = k0; k < k1; ++k) {
+        const unsigned p = w.begin + 2 * k;
+        // The next pair's loads, and the metadata of the one after it. Past the last pair the source is
+        // out of range, so that the wave does not wait for rows it has no use for at its end.
+        const unsigned id = pipe.ahead.id | (k < lastPair ? 0u : 0xFFFFFFFFu);
+        const MetaPair next = ld.meta2(p + 4, last, lane);
+        const float scaleAhead = ld.scale(id);
+        float vn[kValues];
+        loadValues(pipe.ahead, p + 2, vn);
+        gatherPair<S>(ld, w, id, k + 1);
+        stage(v, pipe.scale, p);
+        const unsigned x = at.x + (k & 1u) * 2 * S * 1024;
+        if constexpr (Shared && S == 1) { // eight values a lane in flight: no registers for a pair's operands
+            Operands<1, 1> o;
+            readPanel<0, kYounger>(o, at, x);
+            multiply<1, 1>(o, acc);
+            readPanel<1, kYounger>(o, at, x);
+            multiply<1, 1>(o, acc);
+        } else {
+            Operands<S, 2> o;
+            readPair<S, kYounger>(o, at, x);
+            multiply<S, 2>(o, acc);
+        }
+#pragma unroll
+        for (unsigned j = 0; j < kValues; ++j) v[j] = vn[j];
+        pipe.scale = scaleAhead;
+        pipe.ahead = next;
+    }
+}
+
+// A wave's panels, pair by pair from its first: exclusive pairs, then (from the pair that holds the first
+// shared panel) pairs of any kind. The pipeline runs through: the first shared pair's X, scales and
+// successor's metadata are loaded by the last exclusive step.
+template <unsigned S>
+__device__ __forceinline__ void walkAllPairs(Loader<kBuffer>& ld, TaskWalk& w, const GroupBounds& bounds,
+                                             unsigned exclusive, const MetaPair& first,
+                                             f32x16 (&acc)[4 * S]) {
+    const unsigned pairs = (w.end - w.begin + 1) / 2;
+    PairPipe pipe;
+    pipe.ahead = ld.meta2(w.begin + 2, w.end - 1, w.lane);
+    __builtin_amdgcn_sched_barrier(0);
+    ld.startTask({first.id, first.mask, first.base});
+    pipe.scale = ld.scale(first.id);
+    gatherPair<S>(ld, w, first.id, 0);
+    if (exclusive) walkPairs<false, S>(ld, w, bounds, 0, exclusive, pairs - 1, first, pipe, acc);
+    if (exclusive < pairs) {
+        const MetaPair cur = exclusive ? ld.meta2(w.begin + 2 * exclusive, w.end - 1, w.lane) : first;
+        walkPairs<true, S>(ld, w, bounds, exclusive, pairs, pairs - 1, cur, pipe, acc);
+    }
+    // The loads past the end have to land before their ring slots hold anything else.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
 template <unsigned S, class Ld>
@@ -823,7 +1041,12 @@ __device__ __forceinline__ void walkTask(Ld& ld, const unsigned* offsets, unsign
                                          unsigned end, unsigned lane, const Lds& lds,
                                          f32x16 (&acc)[4 * S]) {
     if (begin >= end) return;
-    const Meta first = ld.meta8(begin, begin, lane);
+    const auto first = [&] {
+        if constexpr (Ld::kWide)
+            return ld.meta8(begin, begin, lane);
+        else
+            return ld.meta2(begin, end - 1, lane);
+    }();
     // An opaque definition keeps the mask in one VGPR for the whole walk instead of a
     // rematerialised literal per use.
     unsigned keep;
@@ -832,11 +1055,17 @@ __device__ __forceinline__ void walkTask(Ld& ld, const unsigned* offsets, unsign
     // %0 is written before %2 is read again: early-clobber, so it never shares the input's register.
     asm("v_and_b32 %0, 31, %2\n\tv_lshrrev_b32 %1, 5, %2" : "=&v"(mh.m), "=v"(mh.h) : "v"(lane));
     TaskWalk w{offsets, begin, end, lane, lds, 0u, keep, mh};
-    auto clipLo = [&](unsigned t) { return max(offsets[t], begin); };
-    auto clipHi = [&](unsigned t) { return min(offsets[t], end); };
     const GroupBounds bounds{offsets[2], offsets[3], offsets[4]};
-    walkPanels<false, S>(ld, w, bounds, clipLo(1), clipHi(5), first, acc);
-    walkPanels<true, S>(ld, w, bounds, clipLo(5), clipHi(16), first, acc);
+    // Exclusive pairs; from the pair with the first shared panel on, pairs of any kind.
+    const unsigned pairs = (end - begin + 1) / 2, shared = offsets[5];
+    const unsigned exclusive = shared >= end ? pairs : (max(shared, begin) - begin) / 2;
+    if constexpr (Ld::kWide) {
+        const unsigned split = min(begin + 2 * exclusive, end);
+        walkPanels<false, S>(ld, w, bounds, begin, split, first, acc);
+        walkPanels<true, S>(ld, w, bounds, split, end, first, acc);
+    } else {
+        walkAllPairs<S>(ld, w, bounds, exclusive, first, acc);
+    }
     waveSync();
 #pragma unroll 1
     for (unsigned i = 0; i < w.redoCount; ++i) {
@@ -926,6 +1155,11 @@ __device__ __forceinline__ unsigned equalBound(unsigned tasks, unsigned x) {
 // end anyway, so the order inside it leaves the L2 sharing of the in-order walk in place.
 constexpr unsigned kTailWindow = 512;
 
+// Whether a task of p panels is in size class c (1..3) or above.
+__device__ __forceinline__ unsigned sizeClass(unsigned p, unsigned c) {
+    return c == 1 ? p >= 96 : c == 2 ? p >= 192 : p >= 288;
+}
+
 // Task at position r (r < n <= kTailWindow) of the window [w0, w0 + n) in size-class order. One
 // wave, all lanes active; every wave computes the same permutation of the window. The sizes of the
 // window's tasks are loaded once (lane L: tasks L, L + 64, ...; all loads in flight together); per 64
@@ -949,7 +1183,7 @@ __device__ __forceinline__ unsigned tailTask(const Sw32Task* tasks, unsigned w0,
         atLeast[ch][0] = in == kWave ? ~std::uint64_t(0) : (std::uint64_t(1) << in) - 1;
 #pragma unroll
         for (unsigned c = 1; c < 4; ++c)
-            atLeast[ch][c] = __builtin_amdgcn_ballot_w64(panels[ch] >= 96 * c) & atLeast[ch][0];
+            atLeast[ch][c] = __builtin_amdgcn_ballot_w64(sizeClass(panels[ch], c)) & atLeast[ch][0];
 #pragma unroll
         for (unsigned c = 0; c < 4; ++c) counts[c] += unsigned(__builtin_popcountll(atLeast[ch][c]));
     }
@@ -1113,11 +1347,9 @@ __device__ __forceinline__ void mergeSlice(const KernelArgs& a, const Sw32Task& 
 // LDS of one wave's walk.
 template <unsigned S>
 struct WaveLds {
-    static constexpr unsigned kAreas = S == 1 ? 1 : 2; // F256 computes its panels in pairs
-    alignas(16) _Float16 table16[256 * kAreas];
-    alignas(16) float table32[256];
-    alignas(16) u32x4 xtile[kAreas * 64 * S];
-    alignas(16) float mant[8 * kAreas];
+    alignas(16) u32x4 xtile[4 * 64 * S]; // walkPairs: a ring of two pairs; walkPanels: one pair
+    alignas(16) _Float16 table16[512];
+    alignas(16) float mant[16];
     alignas(16) unsigned short redo[384];
 };
 
@@ -1192,13 +1424,15 @@ __device__ __forceinline__ void runTask(const KernelArgs& a, unsigned taskIndex)
     const unsigned sw = task.sw;
     unsigned lo = task.begin, hi = task.end;
     if constexpr (Waves > 1) {
-        const std::uint64_t n = hi - lo;
-        lo = task.begin + unsigned(n * wave / Waves);
-        hi = task.begin + unsigned(n * (wave + 1) / Waves);
+        const unsigned pairs = (hi - lo + 1) / 2; // whole pairs, except the last one of an odd task
+        lo = task.begin + 2 * (pairs * wave / Waves);
+        hi = min(task.end, task.begin + 2 * (pairs * (wave + 1) / Waves));
     }
     Loader<Addr> ld(a, lo, hi, Features);
     WaveLds<S>& mem = reinterpret_cast<WaveLds<S>*>(shared)[wave];
-    const Lds lds{mem.table16, mem.table32, mem.xtile, mem.mant, mem.redo};
+    // The FP32 path's table lies behind the one panel of X it uses, after the walk.
+    const Lds lds{mem.table16, reinterpret_cast<float*>(mem.xtile + 128 * S), mem.xtile, mem.mant,
+                  mem.redo};
 
     f32x16 acc[4 * S];
 #pragma unroll
@@ -1289,9 +1523,10 @@ struct TaskClock {
 };
 
 // F128: four waves per SIMD; the 64 accumulators live in ordinary VGPRs and the kernel fits 128
-// registers.
+// registers. The 64-bit-addressed instances hold a pair's operands and their stages in registers and run
+// three (2.45M rows through the 64-bit instance: 3,188 us as one panel at a time and four waves, 3,179).
 template <unsigned Addr, unsigned Waves = 1>
-__global__ __launch_bounds__(kWave * Waves) __attribute__((amdgpu_waves_per_eu(4, 8))) void
+__global__ __launch_bounds__(kWave * Waves) __attribute__((amdgpu_waves_per_eu(Addr == kBuffer ? 4 : 3, 8))) void
 spmmInt8Kernel128(KernelArgs a) {
     TaskClock clock;
     unsigned task;

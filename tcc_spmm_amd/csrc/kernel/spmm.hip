@@ -862,14 +862,21 @@ __device__ __forceinline__ void writeEntry(unsigned address, unsigned offset, _F
     asm volatile("ds_write_b16 %0, %1 offset:%2" ::"v"(address), "v"(v), "n"(offset) : "memory");
 }
 
+// The lane's source in each panel of a pair (slot L >> 3), from the pair's sources. Asked for ahead of the
+// pair's other loads, so that their addresses are computed while the permutes are on their way.
+struct PairSources {
+    unsigned id[2];
+    __device__ PairSources(unsigned ids, unsigned lane)
+        : id{lanePermute(ids, lane >> 3), lanePermute(ids, (lane >> 3) + 8)} {}
+};
+
 // Issues a pair's X rows, to ring slots 2 (k & 1) and 2 (k & 1) + 1.
 template <unsigned S>
-__device__ __forceinline__ void gatherPair(const Loader<kBuffer>& ld, const TaskWalk& w, unsigned id,
-                                           unsigned k) {
+__device__ __forceinline__ void gatherPair(const Loader<kBuffer>& ld, const TaskWalk& w,
+                                           const PairSources& from, unsigned k) {
     unsigned row[2];
 #pragma unroll
-    for (unsigned a = 0; a < 2; ++a)
-        row[a] = (lanePermute(id, (w.lane >> 3) + 8 * a) << ld.xShift) + 16 * (w.lane & 7);
+    for (unsigned a = 0; a < 2; ++a) row[a] = (from.id[a] << ld.xShift) + 16 * (w.lane & 7);
     char* slot = reinterpret_cast<char*>(w.lds.xtile) + (k & 1u) * 2 * S * 1024;
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -988,11 +995,13 @@ __device__ __forceinline__ void walkPairs(Loader<kBuffer>& ld, TaskWalk& w, cons
         // The next pair's loads, and the metadata of the one after it. Past the last pair the source is
         // out of range, so that the wave does not wait for rows it has no use for at its end.
         const unsigned id = pipe.ahead.id | (k < lastPair ? 0u : 0xFFFFFFFFu);
+        const PairSources from(id, lane);
+        __builtin_amdgcn_sched_barrier(0);
         const MetaPair next = ld.meta2(p + 4, last, lane);
         const float scaleAhead = ld.scale(id);
         float vn[kValues];
         loadValues(pipe.ahead, p + 2, vn);
-        gatherPair<S>(ld, w, id, k + 1);
+        gatherPair<S>(ld, w, from, k + 1);
         stage(v, pipe.scale, p);
         const unsigned x = at.x + (k & 1u) * 2 * S * 1024;
         if constexpr (Shared && S == 1) { // eight values a lane in flight: no registers for a pair's operands
@@ -1026,7 +1035,7 @@ __device__ __forceinline__ void walkAllPairs(Loader<kBuffer>& ld, TaskWalk& w, c
     __builtin_amdgcn_sched_barrier(0);
     ld.startTask({first.id, first.mask, first.base});
     pipe.scale = ld.scale(first.id);
-    gatherPair<S>(ld, w, first.id, 0);
+    gatherPair<S>(ld, w, PairSources(first.id, w.lane), 0);
     if (exclusive) walkPairs<false, S>(ld, w, bounds, 0, exclusive, pairs - 1, first, pipe, acc);
     if (exclusive < pairs) {
         const MetaPair cur = exclusive ? ld.meta2(w.begin + 2 * exclusive, w.end - 1, w.lane) : first;
@@ -1365,8 +1374,7 @@ struct WaveLds {
 // LDS: [wave][part of the round][piece 0..7][33 x 16 bytes]: piece 2q + h of row r at index r, 33 so
 // that the eight pieces of a row fall into different banks.
 constexpr unsigned kPiece = 33, kPart = 8 * kPiece;
-template <unsigned Waves>
-constexpr unsigned kRoundParts = Waves == 1 ? 1 : 2;
+constexpr unsigned kRoundParts = 2;
 
 template <unsigned Waves>
 __device__ __forceinline__ void taskSync() {
@@ -1379,7 +1387,7 @@ __device__ __forceinline__ void taskSync() {
 template <unsigned S, unsigned Waves, class Store>
 __device__ __forceinline__ void writeTask(const f32x16 (&acc)[4 * S], f32x4* mem, unsigned wave,
                                           unsigned lane, Store store) {
-    constexpr unsigned kParts = kRoundParts<Waves>;
+    constexpr unsigned kParts = kRoundParts;
     const unsigned row = lane & 31, h = lane >> 5;
     forEachIndex<4 * S / kParts>([&](auto round) __attribute__((always_inline)) {
         constexpr unsigned kFirst = decltype(round)::value * kParts;
@@ -1392,16 +1400,26 @@ __device__ __forceinline__ void writeTask(const f32x16 (&acc)[4 * S], f32x4* mem
             mine[P * kPart + (2 * Q + h) * kPiece + row] = partQuad<I, Q>(slice);
         });
         taskSync<Waves>();
-#pragma unroll 1
-        for (unsigned o = wave; o < 4 * kParts; o += Waves) {
-            const unsigned part = o >> 2, g = o & 3, r = lane >> 3, piece = lane & 7;
-            const f32x4* from = mem + part * kPart + ((piece & 3) * 2 + (piece >> 2)) * kPiece + 8 * g + r;
-            f32x4 sum = from[0];
+        constexpr unsigned kMine = Waves >= 4 * kParts ? 1 : 4 * kParts / Waves; // stretches of this wave
+        constexpr unsigned kBatch = kMine < 4 ? kMine : 4; // LDS reads in flight
+        const unsigned r = lane >> 3, piece = lane & 7;
+        const f32x4* from = mem + ((piece & 3) * 2 + (piece >> 2)) * kPiece + r;
 #pragma unroll
-            for (unsigned v = 1; v < Waves; ++v) sum += from[v * kParts * kPart];
-            sum *= 2.0f; // Y / 2 to Y, exact
-            const unsigned at = kFirst + part; // slice at / 4, features 32 (at % 4) .. + 31
-            store(at >> 2, g, r, 32 * (at & 3) + 4 * piece, sum);
+        for (unsigned b = 0; b < kMine; b += kBatch) {
+            f32x4 sum[kBatch];
+#pragma unroll
+            for (unsigned u = 0; u < kBatch; ++u) {
+                const unsigned o = wave + (b + u) * Waves, part = o >> 2, g = o & 3;
+                sum[u] = from[part * kPart + 8 * g];
+#pragma unroll
+                for (unsigned v = 1; v < Waves; ++v) sum[u] += from[(v * kParts + part) * kPart + 8 * g];
+            }
+#pragma unroll
+            for (unsigned u = 0; u < kBatch; ++u) {
+                const unsigned o = wave + (b + u) * Waves, g = o & 3;
+                const unsigned at = kFirst + (o >> 2); // slice at / 4, features 32 (at % 4) .. + 31
+                store(at >> 2, g, r, 32 * (at & 3) + 4 * piece, sum[u] * 2.0f); // Y / 2 to Y, exact
+            }
         }
     });
 }
@@ -1415,7 +1433,7 @@ template <unsigned Features, unsigned Addr, unsigned Waves = 1>
 __device__ __forceinline__ void runTask(const KernelArgs& a, unsigned taskIndex) {
     constexpr unsigned S = Features / kSlice;
     constexpr std::size_t kWalkBytes = sizeof(WaveLds<S>) * Waves;
-    constexpr std::size_t kWriteBytes = std::size_t(Waves) * kRoundParts<Waves> * kPart * 16;
+    constexpr std::size_t kWriteBytes = std::size_t(Waves) * kRoundParts * kPart * 16;
     __shared__ __align__(16) unsigned char shared[kWalkBytes > kWriteBytes ? kWalkBytes : kWriteBytes];
     __shared__ unsigned lastFlag[S];
     const unsigned wave = Waves == 1 ? 0u : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1594,24 +1612,25 @@ std::uint64_t waveSlots(unsigned features) {
 // marked u: short tasks, to which more waves are of least use):
 //
 //   tasks        250   500u   651  1,002 1,000u 2,090  3,135 4,251  8,566 25,076 31,250u 38,196 78,036
-//   F128 1 wave   79   18.9   129    123   20.6   154    152   159    270    490     345  1,147  2,854
-//        2        45   12.6    74     72   15.6    94     76   113    223    461     354  1,133  2,897
-//        4        27   10.6    50     41   14.9    65     74   118    241    545     394  1,182  3,126
-//        8        20   10.8    36     40   22.7    80    105   160    332
-//   F256 1        99   25.2   161    154   27.0   180    169   197    377    784     599  1,774  4,851
-//        2        56   18.8    97     95   22.6   111    116   190    382    849     627  1,767  5,105
-//        4        34   16.3    56     57   29.9   113    144   224    462  1,127     796  1,966  5,708
-//        8        27   24.3    66     74   43.9   164    223   346    711
+//   F128 1 wave   68   17.7   111    105   19.9   137    114   139    244    460     344  1,136  2,808
+//        2        40   13.0    66     62   15.7    82     67   106    212    450     356  1,128  2,801
+//        4        26   11.5    45     35   17.3    62     72   112    231
+//        8        19   13.4    33     40   23.7    80    101   150    312
+//   F256 1        95   25.5   158    149   26.1   174    164   195    367    764     596  1,765  4,734
+//        2        54   19.1    96     83   23.7   105    115   188    381    857     612  1,747  5,017
+//        4        33   18.5    54     57   30.1   113    138   216    447
+//        8        29   24.7    61     74   44.1   165    210   328    669
 //
-// The lines: 8 waves while every wave has a slot (slots / 8 tasks), 4 up to 3/4 slots; then 2 up to
-// 8 tasks per slot at F128 and 4 at F256, where one wave per task has longer walks and fewer fills.
+// The lines: 8 waves while every wave has a slot (slots / 8 tasks; more would cost plans of short tasks
+// what it gains for others), 4 up to 5/8 slots; then 2 up to 8 tasks per slot at F128 and 3 at F256, where
+// one wave per task has longer walks and fewer fills.
 unsigned taskWaves(unsigned taskCount, unsigned features, std::uint64_t slots) {
     if (const unsigned forced = forcedWaves.load()) return forced;
     if (!slots) return 1;
     const std::uint64_t tasks = taskCount;
     if (8 * tasks <= slots) return 8;
-    if (4 * tasks <= 3 * slots) return 4;
-    return tasks <= (features == 128 ? 8 : 4) * slots ? 2u : 1u;
+    if (8 * tasks <= 5 * slots) return 4;
+    return tasks <= (features == 128 ? 8 : 3) * slots ? 2u : 1u;
 }
 
 template <unsigned Features>

@@ -1,7 +1,7 @@
 """Y at both sides of every line of the rule that picks a task's waves and its workgroup order.
 
-With `slots` wave slots, a plan takes 8 waves per task up to slots / 8 tasks, 4 up to 3/4 slots, and 2
-or 1 above; plans that fill at most half of the slots skip the range search and the tail window. Each
+With `slots` wave slots, a plan takes 8 waves per task up to slots / 8 tasks, 4 up to 5/8 slots, and 2
+or 1 above; plans whose waves fill at most 3/4 of the slots skip the range search and the tail window. Each
 plan here has short tasks of few panels (waves without any panel), split SWs (chunks merged by the
 workgroup's waves) and a last SW with missing rows.
 """
@@ -31,8 +31,8 @@ def _matrix(tasks, rng):
 
 
 @pytest.mark.parametrize("feats", [128, 256])
-@pytest.mark.parametrize("num,den,extra", [(1, 32, 0), (1, 16, 0), (1, 16, 1), (1, 8, 0), (1, 8, 1),
-                                           (3, 4, 0), (3, 4, 1)])
+@pytest.mark.parametrize("num,den,extra", [(1, 32, 0), (3, 32, 0), (3, 32, 1), (1, 8, 0), (1, 8, 1),
+                                           (5, 8, 0), (5, 8, 1), (3, 1, 0), (3, 1, 1)])
 def test_spmm_at_the_lines_of_the_waves_rule(oracle, gpu, feats, num, den, extra):
     import torch
     from tcc_spmm_amd.device import TorchDeviceMatrix

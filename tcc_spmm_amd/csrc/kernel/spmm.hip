@@ -752,9 +752,9 @@ __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBound
 // The compiler orders every LDS access it knows of after the last load to LDS, which would empty the
 // pipeline at each pair. So the accesses of the loop (table entries, mantissas and operands) are written
 // out below, and the wait in front of the operand reads is counted by hand: the loop issues its vector
-// memory instructions in a fixed order (the scheduling barriers keep it), a pair's X last, and kYounger
-// of them, the next pair's, follow before it is read. Only added memory instructions, that is spills,
-// could make the count too high, and the build refuses those.
+// memory instructions in a fixed order (the scheduling barriers keep it), a pair's X last, and the
+// kYounger of the next pair follow before it is read. Further ones in between (the bucket bounds of a shared
+// walk, where a bucket ends) only make the wait stricter.
 
 __device__ __forceinline__ unsigned ldsAddress(const void* p) {
     return unsigned(reinterpret_cast<std::uintptr_t>(
@@ -870,6 +870,15 @@ struct PairSources {
         : id{lanePermute(ids, lane >> 3), lanePermute(ids, (lane >> 3) + 8)} {}
 };
 
+// The sources of the pair at panel p, out of range for panels past the wave's end (whose metadata reads as
+// source 0's): their scales read 0 whatever the caller's scales[0], and the wave does not wait at its end
+// for rows it has no use for.
+__device__ __forceinline__ unsigned sourcesBefore(const TaskWalk& w, unsigned ids, unsigned p) {
+    if (__builtin_expect(p + 1 >= w.end, 0))
+        ids |= p >= w.end || (w.lane & 8) != 0 ? 0xFFFFFFFFu : 0u;
+    return ids;
+}
+
 // Issues a pair's X rows, to ring slots 2 (k & 1) and 2 (k & 1) + 1.
 template <unsigned S>
 __device__ __forceinline__ void gatherPair(const Loader<kBuffer>& ld, const TaskWalk& w,
@@ -902,10 +911,10 @@ struct PairPipe {
 };
 
 // The pairs [k0, k1) of a wave's panels [begin, end), all exclusive or of any kind (Shared). `cur` is
-// the metadata of pair k0; pairs after `lastPair` are never computed and load nothing of X.
+// the metadata of pair k0.
 template <bool Shared, unsigned S>
 __device__ __forceinline__ void walkPairs(Loader<kBuffer>& ld, TaskWalk& w, const GroupBounds& bounds,
-                                          unsigned k0, unsigned k1, unsigned lastPair,
+                                          unsigned k0, unsigned k1,
                                           const MetaPair& cur, PairPipe& pipe, f32x16 (&acc)[4 * S]) {
     constexpr unsigned kValues = Shared ? 8 : 2; // A values of a lane per pair: [row group][pass]
     const unsigned lane = w.lane, last = w.end - 1;
@@ -992,9 +1001,8 @@ __device__ __forceinline__ void walkPairs(Loader<kBuffer>& ld, TaskWalk& w, cons
 #pragma unroll 1
     for (unsigned k = k0; k < k1; ++k) {
         const unsigned p = w.begin + 2 * k;
-        // The next pair's loads, and the metadata of the one after it. Past the last pair the source is
-        // out of range, so that the wave does not wait for rows it has no use for at its end.
-        const unsigned id = pipe.ahead.id | (k < lastPair ? 0u : 0xFFFFFFFFu);
+        // The next pair's loads, and the metadata of the one after it.
+        const unsigned id = sourcesBefore(w, pipe.ahead.id, p + 2);
         const PairSources from(id, lane);
         __builtin_amdgcn_sched_barrier(0);
         const MetaPair next = ld.meta2(p + 4, last, lane);
@@ -1034,12 +1042,13 @@ __device__ __forceinline__ void walkAllPairs(Loader<kBuffer>& ld, TaskWalk& w, c
     pipe.ahead = ld.meta2(w.begin + 2, w.end - 1, w.lane);
     __builtin_amdgcn_sched_barrier(0);
     ld.startTask({first.id, first.mask, first.base});
-    pipe.scale = ld.scale(first.id);
-    gatherPair<S>(ld, w, PairSources(first.id, w.lane), 0);
-    if (exclusive) walkPairs<false, S>(ld, w, bounds, 0, exclusive, pairs - 1, first, pipe, acc);
+    const unsigned ids = sourcesBefore(w, first.id, w.begin);
+    pipe.scale = ld.scale(ids);
+    gatherPair<S>(ld, w, PairSources(ids, w.lane), 0);
+    if (exclusive) walkPairs<false, S>(ld, w, bounds, 0, exclusive, first, pipe, acc);
     if (exclusive < pairs) {
         const MetaPair cur = exclusive ? ld.meta2(w.begin + 2 * exclusive, w.end - 1, w.lane) : first;
-        walkPairs<true, S>(ld, w, bounds, exclusive, pairs, pairs - 1, cur, pipe, acc);
+        walkPairs<true, S>(ld, w, bounds, exclusive, pairs, cur, pipe, acc);
     }
     // The loads past the end have to land before their ring slots hold anything else.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");

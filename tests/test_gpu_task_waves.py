@@ -53,3 +53,30 @@ def test_spmm_at_the_lines_of_the_waves_rule(oracle, gpu, feats, num, den, extra
     # magnitudes; over the 7,000 terms of a hub row that is covered by the oracle's conditioned bound.
     st = ofmt.check_full(pk, sc, y.cpu().numpy(), ATOL, RTOL, cond=16.0, threads=8)
     assert st["checked"] == y.numel() and st["bad"] == 0, st
+
+
+@pytest.mark.parametrize("feats", [128, 256])
+@pytest.mark.parametrize("waves", [0, 1, 2])
+def test_spmm_odd_walks_ignore_the_first_source(oracle, gpu, feats, waves):
+    """A walk of an odd number of panels fills its last pair with an empty panel, whose metadata reads as
+    source 0. No row references source 0 here, so its scale and features may be anything."""
+    from tcc_spmm_amd.device import TorchDeviceMatrix, launch_overrides
+    rng = np.random.default_rng(feats + waves)
+    rows, cols = 32 * 9, 600
+    # SW i: rows of one entry each in its first i + 1 slots' worth of sources: 1 to 9 panels, all exclusive
+    lists = [np.zeros(0, np.int64)] * rows
+    for i in range(9):
+        lists[32 * i + (i % 4) * 8] = np.sort(rng.choice(np.arange(1, cols), 8 * (i + 1) - 3, replace=False))
+    off = np.concatenate([[0], np.cumsum([len(c) for c in lists])]).astype(np.uint32)
+    src = np.concatenate(lists).astype(np.uint32)
+    csr = T.make_canonical_csr(rows, cols, off, src, rng.uniform(-1, 1, src.size).astype(np.float32))
+    packed, scale, _, sc, pk = gpu_prepare(features(cols, feats, seed=7), gpu)
+    dm = TorchDeviceMatrix(T.convert_csr_to_sw32(rows, cols, csr), feats, device=gpu)
+    with launch_overrides(task_waves=waves):
+        want = dm.spmm(packed, scale).clone()
+        for bad in (float("nan"), float("inf"), -float("inf")):
+            scale[0] = bad
+            got = dm.spmm(packed, scale)
+            assert bool((got == want).all()), bad
+    ref = oracle.sw32(rows, cols, *csr.views()).spmm_f64(pk, sc)
+    assert np.abs(want.cpu().numpy() - ref).max() < 1e-3

@@ -69,9 +69,10 @@ void launchSpmmInt8NoAlloc(Sw32DeviceView matrix, const std::int8_t* packedX, co
 
 // Forces two launch choices that launchSpmmInt8 otherwise makes by itself, for tests and
 // measurements (no counterpart in the reference). taskWaves: 0 picks the task form from the plan
-// and the GPU (see above), 1 or 2 forces one or two waves per task (two applies to the
+// and the GPU (see above), 1, 2, 4 or 8 forces that many waves per task (more than one applies to the
 // buffer-addressed instance only). forceWide: the 64-bit-addressing instance for any size.
-// Process-wide. The environment variables TCC_SPMM_TASK_WAVES (1 or 2) and TCC_SPMM_FORCE_WIDE
-// give the initial values, read once, at the first launch or the first call of this function.
-// Throws std::invalid_argument for taskWaves > 2. Not to be called while other host threads launch.
+// Process-wide. The environment variables TCC_SPMM_TASK_WAVES (1, 2, 4 or 8; anything else is
+// reported on stderr and means 1) and TCC_SPMM_FORCE_WIDE give the initial values, read once, at the
+// first launch or the first call of this function.
+// Throws std::invalid_argument for other taskWaves. Not to be called while other host threads launch.
 void setSpmmLaunchOverrides(std::uint32_t taskWaves, bool forceWide);

@@ -54,8 +54,8 @@
 #include <atomic>
 #include <cstddef>
 #include <cstdint>
+#include <cstdio>
 #include <cstdlib>
-#include <cstring>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -1587,10 +1587,17 @@ std::once_flag overridesRead;
 std::atomic<unsigned> forcedWaves{0}; // 0: chosen per launch
 std::atomic<bool> forcedWide{false};
 
+bool isTaskForm(std::uint32_t waves) { return waves == 1 || waves == 2 || waves == 4 || waves == 8; }
+
 void readOverridesOnce() {
     std::call_once(overridesRead, [] {
-        if (const char* w = std::getenv("TCC_SPMM_TASK_WAVES"))
-            forcedWaves.store(std::strcmp(w, "2") == 0 ? 2u : 1u);
+        if (const char* w = std::getenv("TCC_SPMM_TASK_WAVES")) {
+            const unsigned waves = w[0] && !w[1] ? unsigned(w[0] - '0') : 0u;
+            if (!isTaskForm(waves))
+                std::fprintf(stderr, "tcc_spmm: TCC_SPMM_TASK_WAVES=%s is not 1, 2, 4 or 8; one wave "
+                                     "per task\n", w);
+            forcedWaves.store(isTaskForm(waves) ? waves : 1u);
+        }
         if (std::getenv("TCC_SPMM_FORCE_WIDE")) forcedWide.store(true);
     });
 }
@@ -1768,8 +1775,8 @@ void launchSpmmInt8(Sw32DeviceView matrix, const std::int8_t* packedX, const flo
 }
 
 void setSpmmLaunchOverrides(std::uint32_t taskWaves, bool forceWide) {
-    if (taskWaves > 2)
-        throw std::invalid_argument("setSpmmLaunchOverrides: taskWaves must be 0, 1 or 2");
+    if (taskWaves && !isTaskForm(taskWaves))
+        throw std::invalid_argument("setSpmmLaunchOverrides: taskWaves must be 0, 1, 2, 4 or 8");
     readOverridesOnce(); // so that a later first launch keeps these rather than the environment's
     forcedWaves.store(taskWaves);
     forcedWide.store(forceWide);

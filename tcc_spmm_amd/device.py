@@ -181,7 +181,7 @@ def launch_spmm_int8_noalloc(view: DeviceView, packed_x: torch.Tensor, scales: t
 @contextlib.contextmanager
 def launch_overrides(task_waves: int = 0, force_wide: bool = False):
     """setSpmmLaunchOverrides (include/spmm.h; no counterpart in the reference) for the body of a
-    with-block, then back to automatic choices: task_waves 0 (automatic), 1 or 2 waves per task;
+    with-block, then back to automatic choices: task_waves 0 (automatic), 1, 2, 4 or 8 waves per task;
     force_wide selects the 64-bit-addressing kernel instance for any size. Process-wide; for tests
     and measurements."""
     check(lib().tcc_set_spmm_launch_overrides(task_waves, int(force_wide)))

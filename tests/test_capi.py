@@ -1,6 +1,9 @@
 """The C-ABI library loads on a CPU-only host and exports every symbol include/*.h declares."""
 import ctypes
+import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -227,11 +230,24 @@ def test_null_outputs_and_arrays_are_rejected():
 
 
 def test_launch_overrides_hook(launch_overrides):
-    """setSpmmLaunchOverrides takes 0 (automatic), 1 or 2 waves per task and rejects other counts;
-    it touches no GPU."""
+    """setSpmmLaunchOverrides takes 0 (automatic), 1, 2, 4 or 8 waves per task and rejects other
+    counts; it touches no GPU."""
     from tcc_spmm_amd._lib import lib
-    for waves in (0, 1, 2):
+    for waves in (0, 1, 2, 4, 8):
         assert lib().tcc_set_spmm_launch_overrides(waves, 0) == 0
     assert lib().tcc_set_spmm_launch_overrides(1, 1) == 0
-    assert lib().tcc_set_spmm_launch_overrides(3, 0) == 1
-    assert b"taskWaves" in lib().tcc_last_error()
+    for waves in (3, 5, 6, 7, 9, 16, 2 ** 32 - 1):
+        assert lib().tcc_set_spmm_launch_overrides(waves, 0) == 1
+        assert b"taskWaves" in lib().tcc_last_error()
+
+
+@pytest.mark.parametrize("value,reported", [("1", False), ("2", False), ("4", False), ("8", False),
+                                            ("0", True), ("3", True), ("16", True), ("", True)])
+def test_task_waves_environment(value, reported):
+    """TCC_SPMM_TASK_WAVES names a task form; another value is reported, not taken for one silently."""
+    code = ("from tcc_spmm_amd._lib import check, lib\n"
+            "check(lib().tcc_set_spmm_launch_overrides(0, 0))\n")
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True,
+                         env=dict(os.environ, TCC_SPMM_TASK_WAVES=value), cwd=ROOT, timeout=120)
+    assert res.returncode == 0, res.stderr
+    assert ("TCC_SPMM_TASK_WAVES" in res.stderr) == reported

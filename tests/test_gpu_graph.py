@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("entry", ["workspace", "noalloc"])
-@pytest.mark.parametrize("feats,waves", [(128, "1"), (128, "2"), (256, "1")])
+@pytest.mark.parametrize("feats,waves", [(128, "1"), (128, "2"), (256, "1"), (256, "2"), (128, "4"), (256, "4"),
+                                         (128, "8"), (256, "8")])
 def test_spmm_replays_from_a_hip_graph(gpu, entry, feats, waves, launch_overrides):
     import torch
     from tcc_spmm_amd.device import TorchDeviceMatrix, launch_spmm_int8_noalloc

@@ -30,7 +30,7 @@ def _many_chunk_csr():
     return rows, cols, offsets, np.concatenate(sources), np.concatenate(values)
 
 
-@pytest.mark.parametrize("waves", ["1", "2"])
+@pytest.mark.parametrize("waves", ["1", "2", "4", "8"])
 @pytest.mark.parametrize("feats", [128, 256])
 def test_merge_of_many_chunks(oracle, gpu, feats, waves, launch_overrides):
     launch_overrides(task_waves=int(waves))

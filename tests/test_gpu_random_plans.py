@@ -1,4 +1,4 @@
-"""Seeded random plans against the oracle, for both task forms and both widths.
+"""Seeded random plans against the oracle, for every task form and both widths.
 
 Each seed draws a matrix shape (ragged row counts, tail SWs), a degree mix (empty rows, short rows,
 rows long enough to split an SW into several tasks, rows touching one row group or several), value
@@ -54,7 +54,7 @@ def _random_csr(seed):
     return rows, cols, offsets, src.astype(np.uint32), val.astype(np.float32)
 
 
-@pytest.mark.parametrize("waves", ["1", "2"])
+@pytest.mark.parametrize("waves", ["1", "2", "4", "8"])
 @pytest.mark.parametrize("seed", range(12))
 def test_random_plans_against_the_oracle(oracle, gpu, seed, waves, launch_overrides):
     launch_overrides(task_waves=int(waves))

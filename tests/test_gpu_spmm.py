@@ -92,11 +92,11 @@ def test_spmm_c2_full(oracle, gpu, feats):
     assert_close(y, y_ref, f"c2 F{feats}")
 
 
-@pytest.mark.parametrize("waves", ["1", "2"])
+@pytest.mark.parametrize("waves", ["1", "2", "4", "8"])
 @pytest.mark.parametrize("feats", [128, 256])
 def test_spmm_both_task_forms(oracle, golden, gpu, feats, waves, launch_overrides):
     """Each task form whatever the launch would pick (forced through setSpmmLaunchOverrides): one wave per task, or
-    the task's panels shared by two waves whose accumulators wave 0 adds in wave order. On the
+    the task's panels shared by two, four or eight waves whose accumulators are added in wave order. On the
     split and bucket-edge golden cases and on c2: Y within tolerance of the oracle, counters back to
     zero (checked by _run), and a repeated launch bitwise identical."""
     launch_overrides(task_waves=int(waves))
@@ -257,18 +257,20 @@ def test_concurrent_launches_with_separate_workspaces(oracle, gpu, feats):
     assert_close(y_serial, y_ref, f"concurrent F{feats}")
 
 
-@pytest.mark.parametrize("form", ["one wave", "two waves", "64-bit", "u16 packed X"])
+@pytest.mark.parametrize("form", ["one wave", "two waves", "four waves", "eight waves", "64-bit",
+                                  "u16 packed X"])
 @pytest.mark.parametrize("feats", [128, 256])
 def test_spmm_float_aligned_output_and_partials(oracle, gpu, feats, form, launch_overrides):
     """Y and the workspace partials need only be float-aligned, as in the reference (it stores single
     floats, src/kernel/spmm_kernel.cuh:236-245): bases 4, 8 and 12 bytes past a 16-byte boundary, for
     either buffer or both, on a plan with split SWs, give Y bitwise equal to the aligned launch, leave
     the floats around Y untouched and the counters at zero; the allocation-free entry point takes
-    such a Y as well. Every kernel instance compiles its own float-wise path: one and two waves per
+    such a Y as well. Every kernel instance compiles its own float-wise path: one to eight waves per
     task, the 64-bit instance, and the u16 instance (packed X 2 bytes past a 16-byte boundary)."""
     import torch
     from tcc_spmm_amd.device import SpmmWorkspace, launch_spmm_int8, launch_spmm_int8_noalloc
-    launch_overrides(task_waves=2 if form == "two waves" else 1, force_wide=form == "64-bit")
+    waves = {"two waves": 2, "four waves": 4, "eight waves": 8}.get(form, 1)
+    launch_overrides(task_waves=waves, force_wide=form == "64-bit")
     c2 = _split_heavy_csr()
     fmt = T.convert_csr_to_sw32(c2.rows, c2.cols, c2)
     assert fmt.partial_count > 0
@@ -419,7 +421,7 @@ def _fallback_entries(csr, scales):
             | (scales[csr.source_ids] < np.float32(2.0 ** -126)))
 
 
-@pytest.mark.parametrize("waves", ["1", "2"])
+@pytest.mark.parametrize("waves", ["1", "2", "4", "8"])
 @pytest.mark.parametrize("feats", [128, 256])
 def test_spmm_fp32_path_for_extreme_magnitudes(oracle, gpu, feats, waves, launch_overrides):
     """A values of 1e4, 1e-7 and 1e-30 and X rows scaled by 1e6, 1e-6 and into the subnormal range
@@ -489,12 +491,12 @@ def _walk_length_csr():
     return T.make_canonical_csr(rows, cols, off, np.array(src, np.uint32), np.array(val, np.float32))
 
 
-@pytest.mark.parametrize("waves", ["1", "2"])
+@pytest.mark.parametrize("waves", ["1", "2", "4", "8"])
 @pytest.mark.parametrize("feats", [128, 256])
 def test_spmm_every_walk_length(oracle, gpu, feats, waves, launch_overrides):
     """Exclusive walks of 1 to 14 panels in every row group and shared walks of 0 to 6: every length
     modulo six of the F256 loop (panels in pairs, a loop of six, a last panel alone) and of the F128
-    loop (pairs of panels), in both task forms (the two-wave form halves each walk)."""
+    loop (pairs of panels), in every task form (more waves cut each walk into as many parts)."""
     launch_overrides(task_waves=int(waves))
     csr = _walk_length_csr()
     fmt = T.convert_csr_to_sw32(csr.rows, csr.cols, csr)
@@ -509,7 +511,7 @@ def test_spmm_every_walk_length(oracle, gpu, feats, waves, launch_overrides):
     _check_windows(oracle, csr, fmt, y, pk, sc, windows, "walk lengths")
 
 
-@pytest.mark.parametrize("waves", ["1", "2"])
+@pytest.mark.parametrize("waves", ["1", "2", "4", "8"])
 @pytest.mark.parametrize("feats", [128, 256])
 def test_spmm_non_finite_scales(oracle, gpu, feats, waves, launch_overrides):
     """Scales of +inf, -inf and NaN (a caller may pass any scales). Such a slot's panel takes the FP32

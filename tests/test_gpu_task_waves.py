@@ -5,10 +5,16 @@ or 1 above; plans whose waves fill at most 3/4 of the slots skip the range searc
 plan here has short tasks of few panels (waves without any panel), split SWs (chunks merged by the
 workgroup's waves) and a last SW with missing rows.
 """
+import hashlib
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
 import tcc_spmm_amd as T
+from conftest import ROOT
 from gpu_cases import ATOL, RTOL, features, gpu_prepare
 
 pytestmark = pytest.mark.gpu
@@ -56,14 +62,14 @@ def test_spmm_at_the_lines_of_the_waves_rule(oracle, gpu, feats, num, den, extra
 
 
 @pytest.mark.parametrize("feats", [128, 256])
-@pytest.mark.parametrize("waves", [0, 1, 2])
+@pytest.mark.parametrize("waves", [0, 1, 2, 4, 8])
 def test_spmm_odd_walks_ignore_the_first_source(oracle, gpu, feats, waves):
     """A walk of an odd number of panels fills its last pair with an empty panel, whose metadata reads as
     source 0. No row references source 0 here, so its scale and features may be anything."""
     from tcc_spmm_amd.device import TorchDeviceMatrix, launch_overrides
     rng = np.random.default_rng(feats + waves)
     rows, cols = 32 * 9, 600
-    # SW i: rows of one entry each in its first i + 1 slots' worth of sources: 1 to 9 panels, all exclusive
+    # SW i: one row of 8 (i + 1) - 3 entries: i + 1 panels of one exclusive bucket
     lists = [np.zeros(0, np.int64)] * rows
     for i in range(9):
         lists[32 * i + (i % 4) * 8] = np.sort(rng.choice(np.arange(1, cols), 8 * (i + 1) - 3, replace=False))
@@ -80,3 +86,34 @@ def test_spmm_odd_walks_ignore_the_first_source(oracle, gpu, feats, waves):
             assert bool((got == want).all()), bad
     ref = oracle.sw32(rows, cols, *csr.views()).spmm_f64(pk, sc)
     assert np.abs(want.cpu().numpy() - ref).max() < 1e-3
+
+
+def test_task_waves_from_the_environment(gpu):
+    """TCC_SPMM_TASK_WAVES=8 is the form that forcing 8 gives, bit for bit (the order of the additions
+    differs between the forms), and not another one."""
+    from tcc_spmm_amd.device import TorchDeviceMatrix, launch_overrides
+    csr = _matrix(64, np.random.default_rng(3))
+    packed, scale, *_ = gpu_prepare(features(csr.cols, 128, seed=3), gpu)
+    dm = TorchDeviceMatrix(T.convert_csr_to_sw32(csr.rows, csr.cols, csr), 128, device=gpu)
+    forms = {}
+    for waves in (1, 2, 4, 8):
+        with launch_overrides(task_waves=waves):
+            forms[waves] = hashlib.sha256(dm.spmm(packed, scale).cpu().numpy().tobytes()).hexdigest()
+    assert len(set(forms.values())) == 4
+    code = """
+import hashlib, sys
+import numpy as np
+sys.path[:0] = ["tests", "."]
+import tcc_spmm_amd as T
+from gpu_cases import features, gpu_prepare
+from tcc_spmm_amd.device import TorchDeviceMatrix
+from test_gpu_task_waves import _matrix
+csr = _matrix(64, np.random.default_rng(3))
+packed, scale, *_ = gpu_prepare(features(csr.cols, 128, seed=3), "cuda")
+dm = TorchDeviceMatrix(T.convert_csr_to_sw32(csr.rows, csr.cols, csr), 128, device="cuda")
+print(hashlib.sha256(dm.spmm(packed, scale).cpu().numpy().tobytes()).hexdigest())
+"""
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, cwd=ROOT,
+                         env=dict(os.environ, TCC_SPMM_TASK_WAVES="8"), timeout=100)
+    assert res.returncode == 0, res.stderr
+    assert res.stdout.split()[-1] == forms[8]

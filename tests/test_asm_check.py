@@ -1,6 +1,7 @@
 """The build's assembly check (tcc_spmm_amd/asm_check.py) on small hand-written listings, and on
 the kernel source as built here."""
 import pathlib
+import re
 
 from tcc_spmm_amd import asm_check, build
 
@@ -49,6 +50,58 @@ def test_spill_is_flagged():
     assert any("spills" in p for p in problems)
 
 
+def _walk(between, wait="s_waitcnt vmcnt(4)", rows=2):
+    """A loop like the panel walk's: other loads, a pair's X rows to LDS, the wait and the reads of the
+    pair loaded one turn earlier."""
+    row = "\tbuffer_load_dwordx4 v9, s[4:7], 0 offen lds\n"
+    body = row * rows + ".LBB0_1:\n" + between + row * rows
+    body += f"\t;;#ASMSTART\n\t{wait}\n" + "\tds_read_b32 v1, v2\n"
+    return _listing(body + "\t;;#ASMEND\n\ts_cbranch_scc1 .LBB0_1\n")
+
+
+LOAD = "\tbuffer_load_dword v3, v4, s[4:7], 0 offen\n"
+
+
+def test_wait_that_covers_the_pair_passes():
+    assert asm_check.check(_walk(LOAD * 2)) == []
+    assert asm_check.check(_walk(LOAD * 5)) == []                        # stricter than it need be
+    assert asm_check.check(_walk(LOAD, wait="s_waitcnt vmcnt(3)")) == []
+    # loads drained on the way: nothing of the pair is outstanding
+    assert asm_check.check(_walk(LOAD + "\ts_waitcnt vmcnt(0)\n")) == []
+    assert asm_check.check(_walk(LOAD * 2).replace("lds\n", "offset:16\n")) == []  # no loads to LDS
+
+
+def test_wait_one_instruction_short_is_flagged():
+    """A load dropped, merged or sunk below the reads, a wait for fewer, and a row of the next pair that is
+    loaded after the wait."""
+    problems = asm_check.check(_walk(LOAD))
+    assert len(problems) == 1 and "vmcnt(4)" in problems[0]
+    assert len(asm_check.check(_walk(LOAD * 2, wait="s_waitcnt vmcnt(5)"))) == 1
+    assert asm_check.check(_walk(LOAD * 3, rows=1)) == []
+    assert len(asm_check.check(_walk(LOAD * 2, rows=1))) == 1
+
+
+def test_wait_on_a_path_that_skips_a_load_is_flagged():
+    assert len(asm_check.check(_walk("\ts_cbranch_vccnz .LBB0_2\n" + LOAD + ".LBB0_2:\n" + LOAD))) == 1
+
+
+def test_wide_kernel_counts_four_rows_a_pair():
+    listing = _walk(LOAD * 2, wait="s_waitcnt vmcnt(6)", rows=4)
+    assert len(asm_check.check(listing)) == 1
+    assert asm_check.check(listing.replace("10TestKernelEv", "13TestKernel256Ev")) == []
+
+
+def test_operand_reads_without_a_wait_are_flagged():
+    assert len(asm_check.check(_walk(LOAD * 2, wait="s_nop 0"))) == 1
+
+
+def test_address_of_a_load_to_lds_is_a_read():
+    problems = asm_check.check(_listing(
+        "\tv_mfma_f32_32x32x8_f16 v[0:15], v[16:17], v[18:19], v[0:15]\n"
+        "\tbuffer_load_dwordx4 v3, s[4:7], 0 offen lds\n"))
+    assert len(problems) == 1 and "lds" in problems[0]
+
+
 def test_kernel_source_passes(tmp_path):
     """The shipped SpMM kernels compile to clean assembly (this is also part of every build)."""
     build.check_kernel_asm()
@@ -56,3 +109,16 @@ def test_kernel_source_passes(tmp_path):
     assert listing.exists()
     assert asm_check.check(listing.read_text()) == []
     assert pathlib.Path(build.CSRC / "kernel" / "spmm.hip").exists()
+    # The waits of the panel walk are seen: without the pair's last value load (the last indexed load
+    # ahead of its X rows) every kernel that loads X rows to LDS, the buffer-addressed ones, is refused.
+    lines, dropped = [], None
+    for line in listing.read_text().split("\n"):
+        if line.rstrip().endswith(" lds") and dropped is not None:
+            del lines[dropped]
+            dropped = None
+        if line.startswith("\tbuffer_load_dword ") and line.rstrip().endswith("idxen"):
+            dropped = len(lines)
+        lines.append(line)
+    short = [p for p in asm_check.check("\n".join(lines)) if "load to LDS" in p]
+    kernels = {p.split(":")[0] for p in short}
+    assert len(kernels) == 8 and all("ILj0E" in k for k in kernels)

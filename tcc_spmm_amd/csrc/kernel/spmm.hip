@@ -103,7 +103,7 @@ struct KernelArgs {
     float* partials;
     unsigned* counters;
     unsigned rows, cols;
-    unsigned resident; // the whole grid runs at once, with slots to spare (launch)
+    unsigned resident; // the whole grid runs at once (launch): tasks in list order
     unsigned vec4; // y and partials are 16-byte aligned: stores and merge loads of 16 bytes
 #ifdef TCC_SPMM_TIMELINE
     unsigned long long* stamps; // measurement build only: [taskCount][4], see TaskClock
@@ -1256,10 +1256,8 @@ __device__ __forceinline__ bool xcdTask(const KernelArgs& a, unsigned bid, unsig
     const unsigned count = a.m.taskCount, x = bid & 7u, j = bid >> 3;
     const unsigned lane = threadIdx.x & (kWave - 1);
     unsigned lo = equalBound(count, x), hi = equalBound(count, x + 1);
-    // Every workgroup starts at once and a quarter of the wave slots stays free: neither the order nor
-    // the balance decides anything, and finding them takes about 2 us of dependent loads (313 tasks of
-    // 8 waves, F128: 18.3 -> 16.2 us). With the slots nearly full they do matter: three skewed plans of
-    // 450 tasks ran 8-14% slower without them.
+    // Every workgroup starts at once (launch): neither the order nor the balance decides anything, and
+    // finding them takes about 2 us of dependent loads (313 tasks of 8 waves, F128: 18.3 -> 16.2 us).
     if (a.resident) {
         task = lo + j;
         return task < hi;
@@ -1659,7 +1657,15 @@ void launch(KernelArgs args, hipStream_t stream) {
     const bool wide = std::uint64_t(args.cols) * Features > 0xFFFFFF00ull || forcedWide.load();
     const std::uint64_t slots = waveSlots(Features);
     const unsigned waves = misaligned || wide ? 1u : taskWaves(args.m.taskCount, Features, slots);
-    args.resident = 4 * std::uint64_t(args.m.taskCount) * waves <= 3 * slots;
+    // Plans whose workgroups all start at once take their tasks in list order (xcdTask). A quarter of the
+    // slots stays free, since with the slots nearly full the order does matter: three skewed plans of 450
+    // tasks of eight waves ran 8-14% slower without it, and of 1,000 unsplit tasks of four waves 6-14%. Eight
+    // waves of unsplit tasks (none at the 384-panel limit) are short enough to take every slot:
+    // 438-500 tasks, F128, uniform 11.8 -> 9.4 us, power-law 14.8 -> 12.1 and 20.9 -> 20.6, rows sorted by
+    // degree 35.4 -> 34.3; 512 tasks (all slots) 11.9 -> 9.5, but power-law 16.6 -> 17.1; 250 tasks, F256,
+    // 11.7 -> 10.1 to 24.5 -> 23.3.
+    const bool unsplit = args.m.taskCount <= (args.rows + 31) / 32;
+    args.resident = 4 * std::uint64_t(args.m.taskCount) * waves <= (unsplit && waves == 8 ? 4 : 3) * slots;
     const dim3 grid(args.resident ? args.m.taskCount
                                   : args.m.taskCount + 8 * spareWorkgroups(args.m.taskCount));
     auto go = [&](auto kernel, unsigned n) {

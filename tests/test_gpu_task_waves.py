@@ -20,14 +20,15 @@ from gpu_cases import ATOL, RTOL, features, gpu_prepare
 pytestmark = pytest.mark.gpu
 
 
-def _matrix(tasks, rng):
+def _matrix(tasks, rng, hubs=None):
     """A matrix whose plan has exactly `tasks` tasks: SWs of a few panels and, among them, one row of
-    7,000 entries (876 panels, three tasks) per 400 tasks."""
-    hubs = max(1, tasks // 400)
+    7,000 entries (876 panels, three tasks) per 400 tasks, or `hubs` such rows."""
+    hubs = max(1, tasks // 400) if hubs is None else hubs
     sws = tasks - 2 * hubs
     rows, cols = 32 * sws - 5, 9000
     degree = rng.integers(0, 4, rows)
-    degree[rng.choice(sws, hubs, replace=False) * 32 + rng.integers(0, 27, hubs)] = 7000
+    if hubs:
+        degree[rng.choice(sws, hubs, replace=False) * 32 + rng.integers(0, 27, hubs)] = 7000
     lists = [np.sort(rng.choice(cols, d, replace=False)) if d else np.zeros(0, np.int64)
              for d in degree]
     off = np.concatenate([[0], np.cumsum(degree)]).astype(np.uint32)
@@ -58,6 +59,27 @@ def test_spmm_at_the_lines_of_the_waves_rule(oracle, gpu, feats, num, den, extra
     # A sum of n FP32 additions of exact products is off by at most n * 2^-24 of the sum of their
     # magnitudes; over the 7,000 terms of a hub row that is covered by the oracle's conditioned bound.
     st = ofmt.check_full(pk, sc, y.cpu().numpy(), ATOL, RTOL, cond=16.0, threads=8)
+    assert st["checked"] == y.numel() and st["bad"] == 0, st
+
+
+@pytest.mark.parametrize("feats", [128, 256])
+@pytest.mark.parametrize("num,den,extra", [(3, 32, 0), (3, 32, 1), (1, 8, 0), (1, 8, 1),
+                                           (3, 16, 0), (3, 16, 1)])
+def test_spmm_unsplit_plans_at_the_lines_of_the_order_rule(oracle, gpu, feats, num, den, extra):
+    """Plans without split SWs take their tasks in list order up to slots / 8 tasks (eight waves each)
+    and, with four waves, up to 3/16 slots; above the lines by ranges and size classes."""
+    import torch
+    from tcc_spmm_amd.device import TorchDeviceMatrix
+    slots = torch.cuda.get_device_properties(gpu).multi_processor_count * 4 * (4 if feats == 128 else 2)
+    tasks = slots * num // den + extra
+    csr = _matrix(tasks, np.random.default_rng(tasks), hubs=0)
+    fmt = T.convert_csr_to_sw32(csr.rows, csr.cols, csr)
+    assert len(fmt.tasks) == tasks and fmt.partial_count == 0
+    packed, scale, _, sc, pk = gpu_prepare(features(csr.cols, feats, seed=tasks), gpu)
+    y = torch.full((csr.rows, feats), float("nan"), device=gpu)
+    TorchDeviceMatrix(fmt, feats, device=gpu).spmm(packed, scale, y)
+    st = oracle.sw32(csr.rows, csr.cols, *csr.views()).check_full(pk, sc, y.cpu().numpy(), ATOL, RTOL,
+                                                                  threads=8)
     assert st["checked"] == y.numel() and st["bad"] == 0, st
 
 

@@ -227,3 +227,12 @@ def test_tail_order_from_nested_masks():
             member = above[c] & ~above[c + 1] if c < 3 else above[c]
             order.append(int(np.flatnonzero(member)[r - (counts[c + 1] if c < 3 else 0)]))
         assert order == list(np.argsort(-_size_class(panels), kind="stable"))
+
+
+def test_list_order_covers_every_task_once():
+    """Plans whose workgroups all start at once launch one workgroup per task: position bid >> 3 of XCD
+    bid & 7's equal-count range, without spares."""
+    for n in list(range(1, 70)) + [255, 256, 257, 1000, 4097]:
+        tasks = [_equal(n, bid & 7) + (bid >> 3) for bid in range(n)]
+        assert sorted(tasks) == list(range(n))
+        assert all(t < _equal(n, (bid & 7) + 1) for bid, t in enumerate(tasks))

@@ -1547,11 +1547,18 @@ struct TaskClock {
 #endif
 };
 
+// Waves per SIMD of an instance, which its registers have to allow. The launch's wave slots follow it: with
+// four for the 64-bit F128 instances, plans that took all of their slots were held to leave some free and went
+// without an order (2,855 power-law tasks 141 -> 124 us; 2,813 uniform ones 35.1 -> 36.4).
+constexpr unsigned wavesPerSimd(unsigned features, unsigned addr) {
+    return features == 256 ? 2 : addr == kBuffer ? 4 : 3;
+}
+
 // F128: four waves per SIMD; the 64 accumulators live in ordinary VGPRs and the kernel fits 128
 // registers. The 64-bit-addressed instances hold a pair's operands and their stages in registers and run
 // three (2.45M rows through the 64-bit instance: 3,188 us as one panel at a time and four waves, 3,179).
 template <unsigned Addr, unsigned Waves = 1>
-__global__ __launch_bounds__(kWave * Waves) __attribute__((amdgpu_waves_per_eu(Addr == kBuffer ? 4 : 3, 8))) void
+__global__ __launch_bounds__(kWave * Waves) __attribute__((amdgpu_waves_per_eu(wavesPerSimd(128, Addr), 8))) void
 spmmInt8Kernel128(KernelArgs a) {
     TaskClock clock;
     unsigned task;
@@ -1567,7 +1574,7 @@ spmmInt8Kernel128(KernelArgs a) {
 // on c3 this moves 18% fewer bytes (33.1 GB against 40.5 GB) and runs 8.6% faster than one wave
 // per (task, slice).
 template <unsigned Addr, unsigned Waves = 1>
-__global__ __launch_bounds__(kWave * Waves) __attribute__((amdgpu_waves_per_eu(2, 8))) void
+__global__ __launch_bounds__(kWave * Waves) __attribute__((amdgpu_waves_per_eu(wavesPerSimd(256, Addr), 8))) void
 spmmInt8Kernel256(KernelArgs a) {
     TaskClock clock;
     unsigned task;
@@ -1613,11 +1620,10 @@ int currentDeviceCus() {
     return cus;
 }
 
-// Wave slots of the current device: CUs x 4 SIMDs x the kernel's waves per SIMD, 4 at F128 and 2 at
-// F256 (0 when unknown).
-std::uint64_t waveSlots(unsigned features) {
+// Wave slots of the current device: CUs x 4 SIMDs x the instance's waves per SIMD (0 when unknown).
+std::uint64_t waveSlots(unsigned features, unsigned addr) {
     const int cus = currentDeviceCus();
-    return cus <= 0 ? 0 : std::uint64_t(cus) * 4 * (features == 128 ? 4 : 2);
+    return cus <= 0 ? 0 : std::uint64_t(cus) * 4 * wavesPerSimd(features, addr);
 }
 
 // Waves per task. Few tasks for the chip: as many waves as keep the chip's slots in use, since the
@@ -1655,8 +1661,9 @@ void launch(KernelArgs args, hipStream_t stream) {
     // can select the 64-bit instance for any size (used by the tests).
     const bool misaligned = reinterpret_cast<std::uintptr_t>(args.packedX) % 16 != 0;
     const bool wide = std::uint64_t(args.cols) * Features > 0xFFFFFF00ull || forcedWide.load();
-    const std::uint64_t slots = waveSlots(Features);
-    const unsigned waves = misaligned || wide ? 1u : taskWaves(args.m.taskCount, Features, slots);
+    const unsigned addr = misaligned ? kGlobalU16 : wide ? kGlobal : kBuffer;
+    const std::uint64_t slots = waveSlots(Features, addr);
+    const unsigned waves = addr == kBuffer ? taskWaves(args.m.taskCount, Features, slots) : 1u;
     // Plans whose workgroups all start at once take their tasks in list order (xcdTask). A quarter of the
     // slots stays free, since with the slots nearly full the order does matter: three skewed plans of 450
     // tasks of eight waves ran 8-14% slower without it, and of 1,000 unsplit tasks of four waves 6-14%. Eight
@@ -1672,9 +1679,9 @@ void launch(KernelArgs args, hipStream_t stream) {
         hipLaunchKernelGGL(kernel, grid, dim3(n * kWave), 0, stream, args);
     };
     if constexpr (Features == 256) {
-        if (misaligned)
+        if (addr == kGlobalU16)
             go(spmmInt8Kernel256<kGlobalU16>, 1);
-        else if (wide)
+        else if (addr == kGlobal)
             go(spmmInt8Kernel256<kGlobal>, 1);
         else if (waves == 8)
             go(spmmInt8Kernel256<kBuffer, 8>, 8);
@@ -1685,9 +1692,9 @@ void launch(KernelArgs args, hipStream_t stream) {
         else
             go(spmmInt8Kernel256<kBuffer>, 1);
     } else {
-        if (misaligned)
+        if (addr == kGlobalU16)
             go(spmmInt8Kernel128<kGlobalU16>, 1);
-        else if (wide)
+        else if (addr == kGlobal)
             go(spmmInt8Kernel128<kGlobal>, 1);
         else if (waves == 8)
             go(spmmInt8Kernel128<kBuffer, 8>, 8);

@@ -1,7 +1,8 @@
 """The build's assembly check (tcc_spmm_amd/asm_check.py) on small hand-written listings, and on
 the kernel source as built here."""
-import pathlib
 import re
+
+import pytest
 
 from tcc_spmm_amd import asm_check, build
 
@@ -102,17 +103,20 @@ def test_address_of_a_load_to_lds_is_a_read():
     assert len(problems) == 1 and "lds" in problems[0]
 
 
-def test_kernel_source_passes(tmp_path):
-    """The shipped SpMM kernels compile to clean assembly (this is also part of every build)."""
+@pytest.fixture(scope="module")
+def listing():
+    """The assembly of the SpMM kernels, compiled and checked as in every build."""
     build.check_kernel_asm()
-    listing = build.BUILD / "spmm-gfx950.s"
-    assert listing.exists()
-    assert asm_check.check(listing.read_text()) == []
-    assert pathlib.Path(build.CSRC / "kernel" / "spmm.hip").exists()
+    return (build.BUILD / "spmm-gfx950.s").read_text()
+
+
+def test_kernel_source_passes(listing):
+    """The shipped SpMM kernels compile to clean assembly (this is also part of every build)."""
+    assert asm_check.check(listing) == []
     # The waits of the panel walk are seen: without the pair's last value load (the last indexed load
     # ahead of its X rows) every kernel that loads X rows to LDS, the buffer-addressed ones, is refused.
     lines, dropped = [], None
-    for line in listing.read_text().split("\n"):
+    for line in listing.split("\n"):
         if line.rstrip().endswith(" lds") and dropped is not None:
             del lines[dropped]
             dropped = None
@@ -122,3 +126,18 @@ def test_kernel_source_passes(tmp_path):
     short = [p for p in asm_check.check("\n".join(lines)) if "load to LDS" in p]
     kernels = {p.split(":")[0] for p in short}
     assert len(kernels) == 8 and all("ILj0E" in k for k in kernels)
+
+
+def test_wave_slots_are_those_of_the_compiled_instances(listing):
+    """The launch prices a plan against CUs x 4 SIMDs x the waves per SIMD it takes an instance to run;
+    the compiled instances run that many."""
+    occupancy = {}
+    for m in re.finditer(r"^_ZN\S*spmmInt8Kernel(\d+)ILj(\d)E[^\s:]*:", listing, re.M):
+        waves = int(re.search(r"^; Occupancy: (\d+)", listing[m.end():], re.M).group(1))
+        occupancy.setdefault((int(m.group(1)), int(m.group(2))), set()).add(waves)
+    source = (build.CSRC / "kernel" / "spmm.hip").read_text()
+    rule = re.search(r"constexpr unsigned wavesPerSimd\(.*?return (.*?);", source, re.S).group(1)
+    assert rule == "features == 256 ? 2 : addr == kBuffer ? 4 : 3"
+    assert "waveSlots(Features, addr)" in source
+    want = {(f, a): {2 if f == 256 else 4 if a == 0 else 3} for f in (128, 256) for a in (0, 1, 2)}
+    assert occupancy == want

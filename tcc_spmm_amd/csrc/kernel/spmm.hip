@@ -556,13 +556,34 @@ __device__ __forceinline__ void computePanelF32(const Stage& s, unsigned groups,
 // ------------------------------------------------------------------------------------------------
 // Panel walk
 
-// Row groups of the shared-bucket panels of one task, walked in increasing panel order (bucket slot
-// t covers [bucketOffsets[t], bucketOffsets[t + 1]) of the SW). `groups(p)` must be asked for
-// non-decreasing p.
+// Ends of the exclusive buckets of row groups 0..2 (group 3's is the end of the walk), and the first and
+// the end of the first shared bucket: loaded together, before the walk.
+struct GroupBounds {
+    unsigned b0, b1, b2, shared, sharedEnd;
+    __device__ unsigned end(unsigned g) const {
+        return g == 0 ? b0 : g == 1 ? b1 : g == 2 ? b2 : 0xFFFFFFFFu;
+    }
+    // Row group of panel p (the ends do not decrease).
+    __device__ unsigned of(unsigned p) const {
+        return unsigned(p >= b0) + unsigned(p >= b1) + unsigned(p >= b2);
+    }
+    // Row groups of a mixed walk's first panel p, the only one of it that may be exclusive.
+    template <class Cursor>
+    __device__ unsigned firstGroups(Cursor& bucket, unsigned p) const {
+        return p < shared ? 1u << of(p) : bucket.groups(p);
+    }
+};
+
+// Row groups of the panels of one task from the first shared one on, walked in increasing panel order
+// (bucket slot t covers [bucketOffsets[t], bucketOffsets[t + 1]) of the SW). `groups(p)` must be asked
+// for non-decreasing p. A load for each bucket passed (empty ones too), which the wave waits for with every
+// load in flight; none for the first bucket.
 struct BucketCursor {
     const unsigned* offsets; // bucketOffsets of the SW (17 entries)
     unsigned t, end;         // current bucket slot and its end panel
 
+    __device__ BucketCursor(const unsigned* bucketOffsets, const GroupBounds& b)
+        : offsets(bucketOffsets), t(5), end(b.sharedEnd) {}
     __device__ unsigned groups(unsigned p) {
         while (p >= end) {
             ++t;
@@ -599,18 +620,6 @@ __device__ __forceinline__ void flagRedo(TaskWalk& w, unsigned panel, bool redo)
     }
 }
 
-// Ends of the exclusive buckets of row groups 0..2 (group 3's is the end of the walk).
-struct GroupBounds {
-    unsigned b0, b1, b2;
-    __device__ unsigned end(unsigned g) const {
-        return g == 0 ? b0 : g == 1 ? b1 : g == 2 ? b2 : 0xFFFFFFFFu;
-    }
-    // Row group of panel p (the ends do not decrease).
-    __device__ unsigned of(unsigned p) const {
-        return unsigned(p >= b0) + unsigned(p >= b1) + unsigned(p >= b2);
-    }
-};
-
 // Row group of the exclusive panels of one task, walked in increasing panel order. Wave-uniform, in
 // scalar registers: a panel inside the current bucket costs one compare and an untaken branch.
 struct GroupCursor {
@@ -635,7 +644,7 @@ __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBound
     const unsigned n = hi - lo, lane = w.lane, last = w.end - 1;
     // The loads' side of a bucket change: to be called before the loads of panel p, for increasing p.
     // Returns a shared panel's row groups.
-    BucketCursor bucket{w.offsets, 1, Shared ? w.offsets[2] : 0u};
+    BucketCursor bucket(w.offsets, bounds);
     GroupCursor loads{0, 0};
     const unsigned bit0 = 1u << (lane >> 3);
     RowBit rowBit{};
@@ -687,7 +696,7 @@ __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBound
     if (lo == w.begin) ld.startTask(first);
     Stage sa, sb, sc;
     {
-        const unsigned g0 = enter(lo);
+        const unsigned g0 = Shared ? bounds.firstGroups(bucket, lo) : enter(lo);
         loadStage<Shared, S>(ld, first, rowBit, g0, lane, sa);
         const unsigned g1 = enter(lo + 1);
         loadStage<Shared, S>(ld, next, rowBit, g1, lane, sb);
@@ -753,8 +762,9 @@ __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBound
 // pipeline at each pair. So the accesses of the loop (table entries, mantissas and operands) are written
 // out below, and the wait in front of the operand reads is counted by hand: the loop issues its vector
 // memory instructions in a fixed order (the scheduling barriers keep it), a pair's X last, and the
-// kYounger of the next pair follow before it is read. Further ones in between (the bucket bounds of a shared
-// walk, where a bucket ends) only make the wait stricter.
+// kYounger of the next pair follow before it is read. Where a shared walk passes a bucket's end, the loads of the
+// next buckets' bounds come in between, and waiting for them empties the pipeline. The build checks the count on
+// every path of the compiled kernels.
 
 __device__ __forceinline__ unsigned ldsAddress(const void* p) {
     return unsigned(reinterpret_cast<std::uintptr_t>(
@@ -928,16 +938,16 @@ __device__ __forceinline__ void walkPairs(Loader<kBuffer>& ld, TaskWalk& w, cons
 
     // A pair's A values. Exclusive: `bits` is the lane's row bit of pass 0.
     PairCursor loads;
-    BucketCursor bucket{w.offsets, 1, Shared ? w.offsets[2] : 0u};
+    BucketCursor bucket(w.offsets, bounds);
     unsigned bits = 0;
-    auto loadValues = [&](const MetaPair& m, unsigned p, float (&v)[kValues]) __attribute__((always_inline)) {
+    auto loadValues = [&](const MetaPair& m, unsigned p, float (&v)[kValues], auto first) __attribute__((always_inline)) {
         unsigned present = m.mask;
         if constexpr (Shared) {
             // Only the row groups of the panel's bucket.
             auto bytes = [](unsigned g) {
                 return (g & 1u) * 0xFFu | (g & 2u) * 0x7F80u | (g & 4u) * 0x3FC000u | (g & 8u) * 0x1FE00000u;
             };
-            const unsigned g0 = bytes(bucket.groups(min(p, last)));
+            const unsigned g0 = bytes(decltype(first)::value ? bounds.firstGroups(bucket, p) : bucket.groups(min(p, last)));
             const unsigned g1 = bytes(bucket.groups(min(p + 1, last)));
             present &= second ? g1 : g0;
         } else if (loads.changes(p)) {
@@ -997,7 +1007,7 @@ __device__ __forceinline__ void walkPairs(Loader<kBuffer>& ld, TaskWalk& w, cons
     };
 
     float v[kValues];
-    loadValues(cur, w.begin + 2 * k0, v);
+    loadValues(cur, w.begin + 2 * k0, v, std::true_type{});
 #pragma unroll 1
     for (unsigned k = k0; k < k1; ++k) {
         const unsigned p = w.begin + 2 * k;
@@ -1008,7 +1018,7 @@ __device__ __forceinline__ void walkPairs(Loader<kBuffer>& ld, TaskWalk& w, cons
         const MetaPair next = ld.meta2(p + 4, last, lane);
         const float scaleAhead = ld.scale(id);
         float vn[kValues];
-        loadValues(pipe.ahead, p + 2, vn);
+        loadValues(pipe.ahead, p + 2, vn, std::false_type{});
         gatherPair<S>(ld, w, from, k + 1);
         stage(v, pipe.scale, p);
         const unsigned x = at.x + (k & 1u) * 2 * S * 1024;
@@ -1073,10 +1083,10 @@ __device__ __forceinline__ void walkTask(Ld& ld, const unsigned* offsets, unsign
     // %0 is written before %2 is read again: early-clobber, so it never shares the input's register.
     asm("v_and_b32 %0, 31, %2\n\tv_lshrrev_b32 %1, 5, %2" : "=&v"(mh.m), "=v"(mh.h) : "v"(lane));
     TaskWalk w{offsets, begin, end, lane, lds, 0u, keep, mh};
-    const GroupBounds bounds{offsets[2], offsets[3], offsets[4]};
+    const GroupBounds bounds{offsets[2], offsets[3], offsets[4], offsets[5], offsets[6]};
     // Exclusive pairs; from the pair with the first shared panel on, pairs of any kind.
-    const unsigned pairs = (end - begin + 1) / 2, shared = offsets[5];
-    const unsigned exclusive = shared >= end ? pairs : (max(shared, begin) - begin) / 2;
+    const unsigned pairs = (end - begin + 1) / 2;
+    const unsigned exclusive = bounds.shared >= end ? pairs : (max(bounds.shared, begin) - begin) / 2;
     if constexpr (Ld::kWide) {
         const unsigned split = min(begin + 2 * exclusive, end);
         walkPanels<false, S>(ld, w, bounds, begin, split, first, acc);

@@ -139,3 +139,45 @@ print(hashlib.sha256(dm.spmm(packed, scale).cpu().numpy().tobytes()).hexdigest()
                          env=dict(os.environ, TCC_SPMM_TASK_WAVES="8"), timeout=100)
     assert res.returncode == 0, res.stderr
     assert res.stdout.split()[-1] == forms[8]
+
+
+def _shared_entry_csr():
+    """22 SWs: SW i has i % 3 and (i // 3) % 2 exclusive panels of two row groups (its shared part starts in
+    the middle of a pair or not), then 1 to 3 panels in each of two shared buckets, the first of them bucket
+    i % 11 of the eleven (those before it empty), the second further on or missing."""
+    from itertools import combinations
+    rng = np.random.default_rng(23)
+    shared = [sum(1 << g for g in c) for n in (2, 3, 4) for c in combinations(range(4), n)]
+    rows_of = []
+    nxt = 0
+    for i in range(22):
+        panels = {1 << (i % 4): i % 3, 1 << ((i + 1) % 4): (i // 3) % 2, shared[i % 11]: 1 + i % 3}
+        if i % 11 < 10:
+            panels[shared[10 - (i * 7) % (10 - i % 11)]] = 1 + (i + 1) % 3
+        lists = [[] for _ in range(32)]
+        for mask, n in panels.items():
+            for s in range(nxt, nxt + 8 * n):
+                for g in range(4):
+                    if mask >> g & 1:
+                        lists[8 * g + int(rng.integers(0, 8))].append(s)
+            nxt += 8 * n
+        rows_of += lists
+    off = np.concatenate([[0], np.cumsum([len(r) for r in rows_of])]).astype(np.uint32)
+    src = np.concatenate([np.sort(np.array(r, np.uint32)) for r in rows_of])
+    return T.make_canonical_csr(len(rows_of), nxt, off, src, rng.uniform(0.1, 1, src.size).astype(np.float32))
+
+
+@pytest.mark.parametrize("feats", [128, 256])
+@pytest.mark.parametrize("waves,wide", [(1, False), (2, False), (4, False), (8, False), (1, True)])
+def test_spmm_walks_that_enter_the_shared_buckets_anywhere(oracle, gpu, feats, waves, wide):
+    from tcc_spmm_amd.device import TorchDeviceMatrix, launch_overrides
+    csr = _shared_entry_csr()
+    fmt = T.convert_csr_to_sw32(csr.rows, csr.cols, csr)
+    per = np.diff(fmt.bucket_offsets.reshape(-1, 17).astype(np.int64), axis=1)
+    assert set((per[:, 5:] > 0).argmax(axis=1)) == set(range(11))  # every bucket is some SW's first shared one
+    assert set(per[:, 1:5].sum(axis=1) % 2) == {0, 1}
+    packed, scale, _, sc, pk = gpu_prepare(features(csr.cols, feats, seed=5), gpu)
+    with launch_overrides(task_waves=waves, force_wide=wide):
+        y = TorchDeviceMatrix(fmt, feats, device=gpu).spmm(packed, scale).cpu().numpy()
+    st = oracle.sw32(csr.rows, csr.cols, *csr.views()).check_full(pk, sc, y, ATOL, RTOL, threads=8)
+    assert st["checked"] == y.size and st["bad"] == 0, st

@@ -95,6 +95,16 @@ __device__ __forceinline__ float roundTf32(float v) {
     return __uint_as_float((__float_as_uint(v) + 0x1000u) & 0xFFFFE000u);
 }
 
+// f(0), ..., f(N - 1), the index a constant.
+template <class F, unsigned... I>
+__device__ __forceinline__ void forEachIndex(std::integer_sequence<unsigned, I...>, F f) {
+    (f(std::integral_constant<unsigned, I>{}), ...);
+}
+template <unsigned N, class F>
+__device__ __forceinline__ void forEachIndex(F f) {
+    forEachIndex(std::make_integer_sequence<unsigned, N>{}, f);
+}
+
 struct KernelArgs {
     Sw32DeviceView m;
     const std::int8_t* packedX;
@@ -1146,15 +1156,6 @@ __device__ __forceinline__ f32x4 partQuad(const f32x16 (&acc)[4]) {
         v[t] = acc[(rem & 1u) * 2 + hiHalf][4 * I + (rem >> 1)];
     }
     return v;
-}
-
-template <class F, unsigned... I>
-__device__ __forceinline__ void forEachIndex(std::integer_sequence<unsigned, I...>, F f) {
-    (f(std::integral_constant<unsigned, I>{}), ...);
-}
-template <unsigned N, class F>
-__device__ __forceinline__ void forEachIndex(F f) {
-    forEachIndex(std::make_integer_sequence<unsigned, N>{}, f);
 }
 
 // Workgroup -> task. Workgroups are dispatched to the 8 XCDs round-robin by id, and XCD x walks

@@ -41,10 +41,11 @@
 // F256 two.
 //
 // Split SWs (reference src/kernel/spmm_kernel.cuh:228-282): a split task stores its row groups of
-// `task.mask` as 8-row partial tiles [tile][8][F]; lane 0 then takes, per slice, an agent-scope
-// acq_rel wrapping ticket on counters[sw * (F/128) + slice] with limit chunks - 1, so the counter
-// returns to zero by itself; the task whose ticket is chunks - 1 merges all partial tiles of the SW's
-// slice in partialIds order starting from 0.0f and writes Y. No float atomics, no spin-waits.
+// `task.mask` as 8-row partial tiles [tile][8][F]; one lane then publishes them with one agent-scope
+// release fence and takes, per slice, a relaxed wrapping ticket on counters[sw * (F/128) + slice] with
+// limit chunks - 1, so the counter returns to zero by itself; the task whose ticket is chunks - 1, after
+// an acquire fence, merges all partial tiles of the SW's slice in partialIds order starting from 0.0f
+// and writes Y. No float atomics, no spin-waits.
 #include "spmm.h"
 #include "hip_support.h"
 
@@ -264,25 +265,20 @@ struct Loader {
     }
 };
 
-// Panel kinds: exclusive (a bucket of one row group, known per panel from the bucket bounds) and
-// shared (a bucket of several row groups, `groups`).
-struct Stage {     // one panel, ready to compute
+// One panel of walkPanels or of the FP32 pass, ready to compute. Panel kinds: exclusive (a bucket of one
+// row group g, known per panel from the bucket bounds; walkPanels only) and shared (a bucket of several row
+// groups, `groups`, or any panel taken as one).
+struct Stage {
     float scale;   // lane L: scale of slot L & 7
     float v[4];    // lane L: raw A value of (slot L & 7, row 8g + (L >> 3)); v[0] when exclusive
     unsigned bits; // bit g: that entry is present (wide loader only; narrow reads 0 instead)
     u32x4 x[2];    // 16-byte tile L & 7 of the X row of slot L >> 3, per slice of the wave
 };
 
-// Where an exclusive panel's entries are: lane L's row bit in the slot masks, 1 << (8g + (L >> 3))
-// for the panel's row group g, and the bits below it.
-struct RowBit {
-    unsigned at, below;
-};
-
-// Stage 2 of one panel (exclusive: `rowBit`; shared: row groups `groups`), with the X tiles of the
-// wave's S slices.
+// Loads one panel (exclusive: lane L's row bit in the slot masks, 1 << (8g + (L >> 3)), in `rowBit`;
+// shared: row groups `groups`), with the X tiles of the wave's S slices.
 template <bool Shared, unsigned S, class Ld>
-__device__ __forceinline__ void loadStage(const Ld& ld, const Meta& m, const RowBit& rowBit,
+__device__ __forceinline__ void loadStage(const Ld& ld, const Meta& m, unsigned rowBit,
                                           unsigned groups, unsigned lane, Stage& s) {
     // Padding slots (source UINT32_MAX, metadata 0) have an empty row mask; their scale and X tile
     // read 0 (narrow) or a clamped row (wide), multiplied by A entries that are all 0.
@@ -291,11 +287,10 @@ __device__ __forceinline__ void loadStage(const Ld& ld, const Meta& m, const Row
     constexpr unsigned kCount = Shared ? 4 : 1;
 #pragma unroll
     for (unsigned j = 0; j < kCount; ++j) {
-        const unsigned at = Shared ? 1u << (j * 8 + (lane >> 3)) : rowBit.at;
-        const unsigned below = Shared || Ld::kWide ? at - 1u : rowBit.below;
+        const unsigned at = Shared ? 1u << (j * 8 + (lane >> 3)) : rowBit;
         const bool present = (m.mask & at) != 0 && (!Shared || ((groups >> j) & 1u));
         // The k-th set row bit of a slot owns values[base + k].
-        const unsigned idx = m.base + __popc(m.mask & below);
+        const unsigned idx = m.base + __popc(m.mask & (at - 1u));
         s.v[j] = ld.value(idx, present);
         if constexpr (Ld::kWide) s.bits |= unsigned(present) << j;
     }
@@ -333,8 +328,8 @@ __device__ __forceinline__ f16x2 roundPack(float a, float b) {
     return __builtin_amdgcn_cvt_pkrtz(r[0], r[1]);
 }
 
-// LDS handoff between the lanes of the workgroup's single wave: the wave's LDS operations execute
-// in order, so only the compiler has to be kept from moving memory accesses across this point.
+// LDS handoff between the lanes of one wave: a wave's LDS operations execute in order, so only the
+// compiler has to be kept from moving memory accesses across this point.
 __device__ __forceinline__ void waveSync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -346,7 +341,7 @@ struct Lds {
     float* table32;    // [32 rows][8 slots] tf32(a) / 2 (FP32 path)
     u32x4* xtile;      // X rows: xTile, or the ring of walkPairs
     float* mant;       // [2 areas][8 slots] scale mantissas of a panel
-    unsigned short* redo; // [384]: offsets (from the task's first panel) of the panels that need
+    unsigned short* redo; // [384]: offsets (from the wave's first panel) of the panels that need
                           // the FP32 path, in the order found (a task has <= 384 panels)
 };
 
@@ -413,7 +408,7 @@ __device__ __forceinline__ unsigned xTile(unsigned slot, unsigned block) {
 // exclusive panel writes only its own row group, whose table entry of this lane is `entry` (the
 // other groups' entries hold 0). Returns whether every entry of the panel has an exact f16 a'
 // (wave-uniform); if not, its table is all zero, so the panel contributes nothing here.
-template <bool Wide, bool Shared, unsigned S>
+template <bool Shared, unsigned S>
 __device__ __forceinline__ bool stagePanel(const Stage& s, unsigned lane, const Lds& lds, unsigned area,
                                            unsigned entry, unsigned keep) {
     // 2^(e + kShift) for the slot's scale s = m * 2^e (m in [0.5, 1)): its exponent bits alone are
@@ -427,7 +422,7 @@ __device__ __forceinline__ bool stagePanel(const Stage& s, unsigned lane, const 
     _Float16 ap[kCount];
 #pragma unroll
     for (unsigned j = 0; j < kCount; ++j) {
-        const float at = stageTf32<Wide>(s, j);
+        const float at = stageTf32<true>(s, j);
         // a' = at x pow2 has at most eleven significant bits, so it is exact in f16 exactly when
         // its conversion is a normal f16: [2^-14, 65504]; larger values (inf included) convert to
         // inf, smaller ones to subnormals or zero. (A product that lands in that range is a normal
@@ -657,13 +652,12 @@ __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBound
     BucketCursor bucket(w.offsets, bounds);
     GroupCursor loads{0, 0};
     const unsigned bit0 = 1u << (lane >> 3);
-    RowBit rowBit{};
+    unsigned rowBit = 0;
     auto enter = [&](unsigned p) __attribute__((always_inline)) {
         if constexpr (Shared) return bucket.groups(min(p, last));
         if (__builtin_expect(p >= loads.end, 0)) {
             loads.advance(bounds, p);
-            rowBit.at = bit0 << (8 * loads.g);
-            rowBit.below = rowBit.at - 1u;
+            rowBit = bit0 << (8 * loads.g);
         }
         return 0u;
     };
@@ -684,7 +678,7 @@ __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBound
                 entry[A] = tableEntry(staged[A].g, lane, A);
             }
         }
-        flagRedo(w, p, !stagePanel<Ld::kWide, Shared, S>(st, lane, w.lds, A, entry[A], w.keep));
+        flagRedo(w, p, !stagePanel<Shared, S>(st, lane, w.lds, A, entry[A], w.keep));
     };
     auto computePair = [&]() __attribute__((always_inline)) {
         if constexpr (Shared && S == 1) { // as walkPairs
@@ -744,7 +738,7 @@ __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBound
     if (r & 1) {
         const Stage odd = r == 1 ? sa : r == 3 ? sc : sb;
         stage(odd, hi - 1, Area0{});
-        stagePanel<Ld::kWide, Shared, S>(Stage{}, lane, w.lds, 1, entry[1], w.keep);
+        stagePanel<Shared, S>(Stage{}, lane, w.lds, 1, entry[1], w.keep);
         computePair();
     }
 }
@@ -1110,7 +1104,7 @@ __device__ __forceinline__ void walkTask(Ld& ld, const unsigned* offsets, unsign
         const unsigned panel = begin + __builtin_amdgcn_readfirstlane(lds.redo[i]);
         const unsigned groups = groupsOf(offsets, panel);
         Stage st;
-        loadStage<true, S>(ld, ld.meta8(panel, panel, lane), RowBit{}, groups, lane, st);
+        loadStage<true, S>(ld, ld.meta8(panel, panel, lane), 0u, groups, lane, st);
         computePanelF32<Ld::kWide, S>(st, groups, lane, lds, acc);
     }
 }

@@ -1,9 +1,10 @@
 """Y at both sides of every line of the rule that picks a task's waves and its workgroup order.
 
-With `slots` wave slots, a plan takes 8 waves per task up to slots / 8 tasks, 4 up to 5/8 slots, and 2
-or 1 above; plans whose waves fill at most 3/4 of the slots skip the range search and the tail window. Each
-plan here has short tasks of few panels (waves without any panel), split SWs (chunks merged by the
-workgroup's waves) and a last SW with missing rows.
+With `slots` wave slots, a plan takes 8 waves per task up to slots / 8 tasks, 4 up to 5/8 slots, 2 up to 8
+slots at F128 and 3 at F256, and 1 above. Plans whose waves fill at most 3/4 of the slots, or all of them with
+8 waves and no split SW, skip the range search and the tail window: the lines are at 3/32 (8 waves) and 3/16
+(4 waves) of the slots. The plans have short tasks of few panels (waves without any panel), split SWs (chunks
+merged by the workgroup's waves) and a last SW with missing rows.
 """
 import hashlib
 import os
@@ -59,6 +60,51 @@ def test_spmm_at_the_lines_of_the_waves_rule(oracle, gpu, feats, num, den, extra
     # A sum of n FP32 additions of exact products is off by at most n * 2^-24 of the sum of their
     # magnitudes; over the 7,000 terms of a hub row that is covered by the oracle's conditioned bound.
     st = ofmt.check_full(pk, sc, y.cpu().numpy(), ATOL, RTOL, cond=16.0, threads=8)
+    assert st["checked"] == y.numel() and st["bad"] == 0, st
+
+
+def _line_matrix(tasks, rng):
+    """A matrix like _matrix's, drawn without a loop over rows: up to three entries per row, and rows of 7,000
+    (the sum over such a row rounds differently in every task form)."""
+    hubs = max(1, tasks // 400)
+    sws = tasks - 2 * hubs
+    rows, cols = 32 * sws - 5, 9000
+    degree = rng.integers(0, 4, rows)
+    hub_rows = rng.choice(sws, hubs, replace=False) * 32 + rng.integers(0, 27, hubs)
+    degree[hub_rows] = 7000
+    off = np.concatenate([[0], np.cumsum(degree)])
+    at = np.arange(off[-1]) - np.repeat(off[:-1], degree)
+    src = np.repeat(rng.integers(0, cols // 3, rows), degree) + cols // 3 * at
+    for r in hub_rows:
+        src[off[r]:off[r] + 7000] = np.sort(rng.choice(cols, 7000, replace=False))
+    return T.make_canonical_csr(rows, cols, off.astype(np.uint32), src.astype(np.uint32),
+                                rng.uniform(-1, 1, src.size).astype(np.float32))
+
+
+@pytest.mark.parametrize("feats,num,den,extra,waves,other", [
+    (f, n, d, e, w, o) for f in (128, 256) for n, d, e, w, o in (
+        (3, 32, 0, 8, 4), (3, 32, 1, 8, 4), (1, 8, 0, 8, 4), (1, 8, 1, 4, 8), (3, 16, 0, 4, 2),
+        (3, 16, 1, 4, 2), (5, 8, 0, 4, 2), (5, 8, 1, 2, 4), (3, 1, 0, 2, 1))
+] + [(256, 3, 1, 1, 1, 2), (128, 3, 1, 1, 2, 1), (128, 8, 1, 0, 2, 1), (128, 8, 1, 1, 1, 2)])
+def test_spmm_takes_the_form_of_the_waves_rule(oracle, gpu, feats, num, den, extra, waves, other):
+    """The launch's own choice is `waves`, and not the form on the line's other side: its Y is that form's bit
+    for bit."""
+    import torch
+    from tcc_spmm_amd.device import TorchDeviceMatrix, launch_overrides
+    slots = torch.cuda.get_device_properties(gpu).multi_processor_count * 4 * (4 if feats == 128 else 2)
+    tasks = slots * num // den + extra
+    csr = _line_matrix(tasks, np.random.default_rng(tasks + feats))
+    fmt = T.convert_csr_to_sw32(csr.rows, csr.cols, csr)
+    assert len(fmt.tasks) == tasks and fmt.partial_count > 0
+    packed, scale, _, sc, pk = gpu_prepare(features(csr.cols, feats, seed=tasks), gpu)
+    dm = TorchDeviceMatrix(fmt, feats, device=gpu)
+    y = dm.spmm(packed, scale)
+    with launch_overrides(task_waves=waves):
+        assert torch.equal(y.view(torch.int32), dm.spmm(packed, scale).view(torch.int32))
+    with launch_overrides(task_waves=other):
+        assert not torch.equal(y.view(torch.int32), dm.spmm(packed, scale).view(torch.int32))
+    st = oracle.sw32(csr.rows, csr.cols, *csr.views()).check_full(pk, sc, y.cpu().numpy(), ATOL, RTOL,
+                                                                  cond=16.0, threads=8)
     assert st["checked"] == y.numel() and st["bad"] == 0, st
 
 

@@ -2,10 +2,11 @@
 //
 // quantize: rows of features % 4 == 0 (16-byte aligned) use 16-byte loads of 4-feature groups and one
 // dword store per 4 quantized bytes: quantizeRowsFit for F <= 256 (one group per lane, several rows
-// per thread held in registers, X read once), quantizeRowsLong above; other widths (5 <= F <= 2048) go
-// through LDS a tile of rows at a time (quantizeTile), the rest one wave per row (quantizeRows). The row's |x| maximum is reduced across its lanes with shuffles, and every element
-// is divided by the scale with the IEEE-correct FP32 divide and rounded half-to-even. Results are bit-identical to reference
-// src/format/int8_quantize.cu:4-25.
+// per thread held in registers, X read once), quantizeRowsLong above; other widths (5 <= F <= 2048) of more
+// than a few thousand rows go through LDS a tile of rows at a time (quantizeTile), the rest one wave per row
+// (quantizeRows). The row's |x| maximum is reduced across its lanes with shuffles, and every element is
+// divided by the scale with the IEEE-correct FP32 divide and rounded half-to-even. Results are bit-identical
+// to reference src/format/int8_quantize.cu:4-25.
 //
 // pack: one thread per 16-byte tile; four v_perm_b32 byte shuffles turn q[0..15] into
 // [q0,q8,q1,q9,...,q7,q15] (reference src/format/pack_int8.cu:6-15). Unaligned buffers use a
@@ -156,8 +157,8 @@ __global__ __launch_bounds__(256) void quantizeRowsLong(const f32x4* __restrict_
 // a width that is not a multiple of 4 is not 16-byte aligned, but a tile is one contiguous stretch: it
 // is copied to LDS with 16-byte loads, the row maxima are taken there (256 / rows threads each), and q is
 // written four bytes at a time across the row ends. Bound by HBM: 300,007 x 50 (75 MB) in 49.9 us with
-// one wave per row and 4-byte loads, 18.7 us with tiles
-// (50,001 x 602: 48.8 -> 36.4; 1,000,003 x 5: 155 -> 8.5).
+// one wave per row and 4-byte loads, 18.6 us with tiles (50,001 x 602: 48.8 -> 37.6; 1,000,003 x 5: 155 ->
+// 8.4).
 constexpr unsigned kTileFeatures = 2048, kTileFloats = 4096;
 
 __global__ __launch_bounds__(256) void quantizeTile(const float* __restrict__ x,
@@ -238,18 +239,37 @@ namespace {
 
 // The quantize kernels for one call: the vector kernels for 16-byte aligned rows of features % 4 ==
 // 0 with a 4-byte aligned output, the tile kernel for other widths of such buffers (at F < 5 four
-// features can span more than two rows; above 2,048 a tile does not fit LDS beside others), the scalar
-// kernel otherwise. `Packed` writes the packed16 layout
-// (features % 16 == 0, checked by the caller).
+// features can span more than two rows; above 2,048 a tile does not fit LDS beside others) unless they have
+// few rows, the scalar kernel otherwise. `Packed` writes the packed16 layout (features % 16 == 0, checked by
+// the caller).
+
+// Whether one wave per row beats tiles. The chip holds 8,192 such waves at once, whose rows then take one
+// memory latency and no barrier; a tile has two barriers, and few rows make few tiles. Well above that the waves
+// come in rounds, narrow rows leave most lanes idle and wide ones loop. Device time in us, wave per row /
+// tiles: F = 13: 4,096 rows 2.4 / 2.8, 8,192 3.0 / 2.8; 33: 10,007 3.4 / 3.6, 12,288 3.7 / 3.3; 50: 4,096 2.4 /
+// 3.3, 16,384 4.3 / 3.9; 127: 12,500 4.7 / 5.0, 16,384 5.4 / 5.3; 201: 4,096 3.4 / 3.9, 12,500 5.9 / 6.3, 20,011 7.9 / 7.7; 257:
+// 12,288 7.4 / 6.8; 511: 2,048 4.4 / 4.0, 6,144 5.4 / 5.9, 10,007 8.6 / 8.6; 599: 8,192 9.4 / 8.4; 767: 1,024
+// 5.4 / 4.1.
+bool fewRows(std::uint32_t sources, std::uint32_t features) {
+    if (features >= 320) return features < 544 && sources > 2048 && sources <= 8192;
+    if (features < 48 || features >= 256) return sources <= (features < 32 ? 7168u : 10240u);
+    return sources <= (features < 96 ? 12288u : 14336u);
+}
+
 template <bool Packed>
 void launchQuantize(const float* x, std::int8_t* out, float* scale, std::uint32_t sources,
                     std::uint32_t features, hipStream_t stream) {
     const bool aligned = reinterpret_cast<std::uintptr_t>(x) % 16 == 0 &&
                          reinterpret_cast<std::uintptr_t>(out) % 4 == 0;
-    if (!Packed && aligned && features % 4 != 0 && features >= 5 && features <= kTileFeatures) {
-        // Tiles of up to 16 KB, and small enough for a block per CU where there are few rows.
+    if (!Packed && aligned && features % 4 != 0 && features >= 5 && features <= kTileFeatures &&
+        !fewRows(sources, features)) {
+        // Tiles of up to 16 KB, and small enough for a block per CU where there are few rows, or two or four,
+        // since one block alone waits through its copy and its barriers (one, two, four: 16,384 x 50 4.7, 3.9,
+        // 4.0 us; 16,384 x 127 6.2, 6.2, 5.3; narrow rows have too little work for that: 16,384 x 13 2.5,
+        // 2.9, 3.3).
+        const unsigned minBlocks = features < 48 ? 256u : features < 96 ? 512u : 1024u;
         unsigned rows = 256;
-        while (rows > 4 && (rows * features > kTileFloats || sources / rows < 256)) rows /= 2;
+        while (rows > 4 && (rows * features > kTileFloats || sources / rows < minBlocks)) rows /= 2;
         const unsigned blocks = unsigned((std::size_t(sources) + rows - 1) / rows);
         const std::size_t lds = (std::size_t(rows) * features + rows + 1) * sizeof(float);
         const unsigned magic = unsigned((std::uint64_t(1) << 32) / features) + 1;

@@ -38,9 +38,10 @@ struct SpmmWorkspace {
 // differs from it. That order is fixed for a given plan and task form: a plan with few tasks for the
 // GPU's wave slots (CU count x 4 SIMDs x 4 waves at F=128, x 2 at F=256) runs two, four or eight
 // waves per task (8 up to an eighth of a task per slot, 4 up to 5/8, 2 up to 8 at F=128 and 3 at
-// F=256), each summing its share of the panels, which orders the additions differently. So Y can differ in the last bits between GPUs
-// with different CU counts (or partition modes), and between the task forms forced by
-// setSpmmLaunchOverrides; repeated launches of one plan on one GPU are bitwise identical.
+// F=256), each summing its share of the panels, which orders the additions differently. So Y can
+// differ in the last bits between GPUs with different CU counts (or partition modes), and between the
+// task forms forced by setSpmmLaunchOverrides; repeated launches of one plan on one GPU are bitwise
+// identical.
 // (reference include/spmm.cuh:15-23)
 void launchSpmmInt8(Sw32DeviceView matrix, const std::int8_t* packedX, const float* scales,
                     float* output, std::uint32_t rows, std::uint32_t cols, std::uint32_t features,

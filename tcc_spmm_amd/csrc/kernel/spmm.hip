@@ -753,10 +753,11 @@ __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBound
 // and table entries, so nothing is moved between lanes to separate the panels; the scale's work is done
 // once per pair; and the pair is one v_mfma_f32_32x32x16_f16 per 32-feature block. X goes straight from
 // memory to LDS (16 bytes per lane), so rows in flight take no registers and F128's pairs fit its 128.
-// Against one panel at a time at F128 and pairs staged panel by panel at F256, X through registers (us):
-// 100K rows F128 74.5 -> 65.2, 262K power law F128 221 -> 213, F256 361 -> 355, 2.45M rows F128
-// 2,872 -> 2,802, F256 4,884 -> 4,761. Loads to LDS alone, with the rest as before, gained nothing
-// (F128 +0.1 to +4%): the depth of the gathers is not what bounds them.
+// Against one panel at a time at F128 and pairs staged panel by panel at F256, X through registers, the two
+// builds timed in turn (us; other sessions differ by a few percent): 100K rows F128 74.5 -> 65.2, 262K power
+// law F128 221 -> 213, F256 361 -> 355, 2.45M rows F128 2,872 -> 2,802, F256 4,884 -> 4,761. Loads to LDS
+// alone, with the rest as before, gained nothing (F128 +0.1 to +4%): with the chip full the depth of the
+// gathers is not what bounds them.
 //
 // LDS of a wave: a ring of two pairs' X rows, [panel & 3][slice][8 slots][128 bytes] as the loads deliver
 // them (lane L: 16 bytes at 16 L); the A table [32 rows][2 halves][2 panels][4 slots]; the mantissas
@@ -766,9 +767,9 @@ __device__ __forceinline__ void walkPanels(Ld& ld, TaskWalk& w, const GroupBound
 // pipeline at each pair. So the accesses of the loop (table entries, mantissas and operands) are written
 // out below, and the wait in front of the operand reads is counted by hand: the loop issues its vector
 // memory instructions in a fixed order (the scheduling barriers keep it), a pair's X last, and the
-// kYounger of the next pair follow before it is read. Where a shared walk passes a bucket's end, the loads of the
-// next buckets' bounds come in between, and waiting for them empties the pipeline. The build checks the count on
-// every path of the compiled kernels.
+// kYounger of the next pair follow before it is read. Where a shared walk passes a bucket's end, the loads of
+// the next buckets' bounds come in between, and waiting for them empties the pipeline. The build checks the
+// count on every path of the compiled kernels.
 
 __device__ __forceinline__ unsigned ldsAddress(const void* p) {
     return unsigned(reinterpret_cast<std::uintptr_t>(
@@ -956,14 +957,16 @@ __device__ __forceinline__ void walkPairs(Loader<kBuffer>& ld, TaskWalk& w, cons
     PairCursor loads;
     BucketCursor bucket(w.offsets, bounds);
     unsigned bits = 0;
-    auto loadValues = [&](const MetaPair& m, unsigned p, float (&v)[kValues], auto first) __attribute__((always_inline)) {
+    auto loadValues = [&](const MetaPair& m, unsigned p, float (&v)[kValues], auto first)
+        __attribute__((always_inline)) {
         unsigned present = m.mask;
         if constexpr (Shared) {
             // Only the row groups of the panel's bucket.
             auto bytes = [](unsigned g) {
                 return (g & 1u) * 0xFFu | (g & 2u) * 0x7F80u | (g & 4u) * 0x3FC000u | (g & 8u) * 0x1FE00000u;
             };
-            const unsigned g0 = bytes(decltype(first)::value ? bounds.firstGroups(bucket, p) : bucket.groups(min(p, last)));
+            const unsigned g0 = bytes(decltype(first)::value ? bounds.firstGroups(bucket, p)
+                                                             : bucket.groups(min(p, last)));
             const unsigned g1 = bytes(bucket.groups(min(p + 1, last)));
             present &= second ? g1 : g0;
         } else if (loads.changes(p)) {
@@ -1122,8 +1125,8 @@ __device__ __forceinline__ void walkTask(Ld& ld, const unsigned* offsets, unsign
         Stage st;
         loadStage<true, S>(ld, ld.meta8(panel, panel, lane), 0u, groups, lane, st);
         // The X rows are asked for before anything waits for the values: left to the scheduler, the table's
-        // entries came first, one more memory latency a panel (12,501 tasks with every panel here, F128 465 -> 419
-        // us, F256 948 -> 854).
+        // entries came first, one more memory latency a panel (12,501 tasks with every panel here, F128 465 ->
+        // 419 us, F256 948 -> 854).
         __builtin_amdgcn_sched_barrier(0);
         computePanelF32<Ld::kWide, S>(st, groups, lane, lds, acc);
     }
@@ -1653,22 +1656,40 @@ std::uint64_t waveSlots(unsigned features, unsigned addr) {
 
 // Waves per task. Few tasks for the chip: as many waves as keep the chip's slots in use, since the
 // longest tasks, not the bandwidth, set the launch time. Measured on MI355X (us; 256 CUs, 4,096 wave slots at
-// F128 and 2,048 at F256; matrices of 20 or 32 entries per row with power-law tails, 8 uniform where
-// marked u: short tasks, to which more waves are of least use):
+// F128 and 2,048 at F256). short: all tasks of 33 panels; equal: all of 130; skewed: power-law rows with
+// communities, 89 panels in the mean and 384 in the longest (SWs split into several tasks):
 //
-//   tasks        250   500u   651  1,002 1,000u 2,090  3,135 4,251  8,566 25,076 31,250u 38,196 78,036
-//   F128 1 wave   68   17.7   111    105   19.9   137    114   139    244    460     344  1,136  2,808
-//        2        40   13.0    66     62   15.7    82     67   106    212    450     356  1,128  2,801
-//        4        26   11.5    45     35   17.3    62     72   112    231
-//        8        19   13.4    33     40   23.7    80    101   150    312
-//   F256 1        95   25.5   158    149   26.1   174    164   195    367    764     596  1,765  4,734
-//        2        54   19.1    96     83   23.7   105    115   188    381    857     612  1,747  5,017
-//        4        33   18.5    54     57   30.1   113    138   216    447
-//        8        29   24.7    61     74   44.1   165    210   328    669
+//   tasks, about        250    500    750  1,000  1,500  2,050  3,150  4,150  6,300 12,600
+//   F128 1 wave  short    16.2   16.7   17.4   18.2   20.7   21.3   31.2   35.5   55.5    121
+//                equal    38.9   41.4   43.1   44.9   52.8   54.2   87.3   96.6    157    338
+//                skewed   96.1    102    103    105    118    128    117    121    167    296
+//   F128 2 waves short    11.1   11.8   12.5   14.2   17.5   21.3   32.2   38.8   55.4    127
+//                equal    23.3   27.9   28.8   31.6   43.8   50.2   78.5    100    149    338
+//                skewed   54.9   60.5   66.2   67.2   59.0   63.7   69.3   83.3    120    268
+//   F128 4 waves short     8.6   10.1   12.0   16.1   22.2   25.8   36.4   44.9   62.2    135
+//                equal    16.2   19.5   24.3   30.5   41.5   52.5   78.5    103    153    343
+//                skewed   35.4   37.6   39.6   37.7   39.7   50.3   71.5   89.4    130    293
+//   F128 8 waves short     8.0   10.6   18.4   22.2   30.5   37.8   55.2   70.1    100    194
+//                equal    13.3   18.6   30.4   36.3   50.9   66.5    106    135    196    410
+//                skewed   26.4   28.0   30.0   38.0   54.5   68.0    100    126    189    401
+//   F256 1 wave  short    22.2   23.4   23.8   24.4   30.0   34.0   59.5   66.7    106    227
+//                equal    53.4   56.9   58.5   59.9   81.5   87.0    160    176    303    623
+//                skewed    131    146    146    147    150    153    161    165    255    448
+//   F256 2 waves short    15.2   18.1   18.6   22.0   36.2   39.6   60.1   75.3    113    235
+//                equal    32.2   42.3   43.9   48.8   87.7   93.8    151    192    291    608
+//                skewed   74.0   90.9    102   81.4   83.6   85.9    119    152    235    459
+//   F256 4 waves short    11.5   16.8   25.0   28.1   38.1   47.8   71.3   90.0    132    262
+//                equal    21.6   30.5   44.0   53.4   75.9   99.8    156    196    308    609
+//                skewed   46.1   47.6   47.4   52.5   73.1   92.5    137    170    273    546
+//   F256 8 waves short    11.3   24.0   33.7   43.5   61.9   80.3    123    159    231    445
+//                equal    18.9   39.2   57.4   76.0    113    150    235    296    434    817
+//                skewed   36.2   41.7   58.7   73.7    113    145    215    276    428    842
 //
-// The lines: 8 waves while every wave has a slot (slots / 8 tasks; more would cost plans of short tasks
-// what it gains for others), 4 up to 5/8 slots; then 2 up to 8 tasks per slot at F128 and 3 at F256, where
-// one wave per task has longer walks and fewer fills.
+// The lines: 8 waves while every wave has a slot (slots / 8 tasks), 4 up to 5/8 slots; then 2 up to 8 tasks
+// per slot at F128 and 3 at F256, where one wave per task has longer walks and fewer fills. The host knows how
+// many tasks there are, not how long they are: short ones would take fewer waves from 1,000 tasks (F128) and
+// 500 (F256) on (750 at F256: 18.6 us with two, 25.0 as chosen), but skewed ones lose more by that than short
+// ones gain (47.4 with four, 102 with two), and equal ones lie between.
 unsigned taskWaves(unsigned taskCount, unsigned features, std::uint64_t slots) {
     if (const unsigned forced = forcedWaves.load()) return forced;
     if (!slots) return 1;

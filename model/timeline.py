@@ -1,6 +1,6 @@
 """Per-task timeline of the SpMM kernel on a synthetic configuration (measurement infrastructure).
 
-    python -m model.timeline c5 [c3 ...]      # on a GPU box; prints a report per config and width
+    python -m model.timeline c5 [c3 ...]      # needs the GPU; prints a report per config and width
 
 The measurement build compiles tcc_spmm_amd/csrc/kernel/spmm.hip with TCC_SPMM_TIMELINE, which makes
 lane 0 of every workgroup store its task's start, the time the task was found, its end

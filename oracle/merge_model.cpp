@@ -7,7 +7,9 @@
 //   - a split task writes its row groups of task.mask as 8-row partial tiles [tile][8][F];
 //   - per 128-feature slice it takes a ticket: an atomic wrapping increment of
 //     counters[sw * F/128 + slice] with limit chunks - 1 (old >= limit ? 0 : old + 1, the
-//     semantics of the GPU's atomic_inc), acquire-release, so the counter returns to zero by itself;
+//     semantics of the GPU's atomic_inc), so the counter returns to zero by itself. The kernel orders
+//     relaxed tickets by one release fence ahead of them and an acquire fence in the merging task; here
+//     the ticket itself is acquire-release, the same guarantee in a form ThreadSanitizer follows;
 //   - the task whose ticket is chunks - 1 merges the slice: per row group, the tiles of the
 //     group's reduction range summed in partialIds order from 0.0f, with the kernel's lane layout
 //     (lane L: row L >> 3, columns slice * 128 + (L & 7) * 4 + 32 j + t), its 64-id chunks and

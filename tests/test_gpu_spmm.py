@@ -16,7 +16,7 @@ from gpu_cases import (ATOL, RTOL, assert_close, assert_close_conditioned, check
 
 pytestmark = pytest.mark.gpu
 
-# Host threads of the full-size checks (a one-GPU box gets a 16-core share of its host).
+# Host threads of the full-size checks.
 CHECK_THREADS = max(1, min(16, os.cpu_count() or 1))
 # Summation-conditioning factor of the checks with cancelling hub rows (assert_close_conditioned).
 COND = 16.0
@@ -426,9 +426,9 @@ def _fallback_entries(csr, scales):
 def test_spmm_fp32_path_for_extreme_magnitudes(oracle, gpu, feats, waves, launch_overrides):
     """A values of 1e4, 1e-7 and 1e-30 and X rows scaled by 1e6, 1e-6 and into the subnormal range
     push some panels onto the FP32 path; Y must still match the oracle (summation-conditioned
-    bound: the rows mix terms across 40 orders of magnitude). At F256 panels go in pairs through
-    one MFMA, so flagged panels sit in either place of a pair and beside unflagged ones, and walks
-    of every length modulo six end with and without an unpaired panel."""
+    bound: the rows mix terms across 40 orders of magnitude). Panels go in pairs through one MFMA, so
+    flagged panels sit in either place of a pair and beside unflagged ones, and walks of every length
+    modulo six end with and without an unpaired panel."""
     launch_overrides(task_waves=int(waves))
     base = T.synth_csr("t3000_24_11")
     rng = np.random.default_rng(12)
@@ -458,7 +458,7 @@ def test_spmm_fp32_path_for_extreme_magnitudes(oracle, gpu, feats, waves, launch
 def _walk_length_csr():
     """14 SWs: SW i has i + 1 panels in the exclusive bucket of row group i % 4 (its last panel short of
     a slot when i % 3 != 0) and (5 i) % 7 panels in the shared bucket of row groups {0, 1}; in SWs 4 to 7
-    one entry in 16 is 1e6 times larger, so some panels, in either place of an F256 pair, take the FP32
+    one entry in 16 is 1e6 times larger, so some panels, in either place of a pair, take the FP32
     path."""
     rng = np.random.default_rng(7)
     nsw, cols = 14, 4096
@@ -495,8 +495,8 @@ def _walk_length_csr():
 @pytest.mark.parametrize("feats", [128, 256])
 def test_spmm_every_walk_length(oracle, gpu, feats, waves, launch_overrides):
     """Exclusive walks of 1 to 14 panels in every row group and shared walks of 0 to 6: every length
-    modulo six of the F256 loop (panels in pairs, a loop of six, a last panel alone) and of the F128
-    loop (pairs of panels), in every task form (more waves cut each walk into as many parts)."""
+    modulo six of the 64-bit-addressed loop (panels in pairs, a loop of six, a last panel alone) and of the
+    buffer-addressed one (pairs of panels), in every task form (more waves cut each walk into as many parts)."""
     launch_overrides(task_waves=int(waves))
     csr = _walk_length_csr()
     fmt = T.convert_csr_to_sw32(csr.rows, csr.cols, csr)

@@ -1,9 +1,9 @@
 """CPU model of the split-SW ticket and merge protocol (oracle/merge_model.cpp), on real plans.
 
 The kernel's end of a split task (tcc_spmm_amd/csrc/kernel/spmm.hip, runTask and mergeSlice;
-reference src/kernel/spmm_kernel.cuh:228-282) is restated for host threads: partial-tile writes, an
-acquire-release wrapping ticket per slice, and the last arriver's merge with the kernel's lane
-layout, 64-id chunks and batches of four tiles. Checked here, without a GPU:
+reference src/kernel/spmm_kernel.cuh:228-282) is restated for host threads: partial-tile writes, a
+wrapping ticket per slice, and the last arriver's merge with the kernel's lane layout, 64-id chunks and
+batches of four tiles. Checked here, without a GPU:
   - lane map: every element of a row group's 8 x 128 block is summed by exactly one lane, from every
     tile of its reduction range exactly once, in partialIds order, and written once (ranges of 1 to
     130 tiles, and every split SW of c5 and of a plan with an SW split 73 ways);
@@ -12,9 +12,9 @@ layout, 64-id chunks and batches of four tiles. Checked here, without a GPU:
     counters are back at zero after every launch, and every merged element is bitwise the serial sum
     of the tile values in partialIds order;
   - ordering: the same runs under ThreadSanitizer report no data race, while a planted mistake
-    (relaxed tickets and no acquire fence) is reported as one. The GPU's agent-scope acquire-release
-    RMW and C++'s acq_rel RMW give the same guarantee here: the last RMW of the release sequence
-    makes every earlier ticket-taker's tile writes visible to the merger.
+    (relaxed tickets and no acquire fence) is reported as one. The GPU's agent-scope release
+    fence, relaxed RMW and acquire fence and the model's acq_rel RMW give the same guarantee here: the
+    last RMW of the release sequence makes every earlier ticket-taker's tile writes visible to the merger.
 """
 import pathlib
 import subprocess

@@ -6,7 +6,8 @@ ranges hold equal task counts unless some XCD would get more than 3% above the m
 then they hold equal panel counts, each boundary clamped to half the spare share from its equal-count
 place, and the grid adds ceil(T / 16) spare workgroups per XCD. The last TAIL_WINDOW tasks of a
 range run longest size class first (tailTask: per 64-lane chunk a ballot count of each class, then
-the k-th member of the chosen class by its rank among the chunk's members). Checked on the synthetic
+the k-th member of the chosen class by its rank among the chunk's members). Plans whose workgroups all start
+at once take their tasks in list order. Checked on the synthetic
 configs and on adversarial lists (all tasks empty, one task holding every panel, heavy skew, random
 sizes), for task counts 1..39 and a few larger ones; the window's order is checked against a stable
 sort by descending class."""
@@ -49,7 +50,8 @@ def _tail_order(cls, w0):
 
 
 def _panel_bound(begin, count, target):
-    """panelBound for one half: 32 probes per step over [l, r], task r known to qualify."""
+    """A search with 32 probes per step over [l, r], task r known to qualify (the kernel's form before
+    BoundSearch, whose steps _bound_search restates)."""
     l, r = 0, count
     while l < r:
         stride = (r - l + 31) // 32
@@ -136,8 +138,8 @@ def test_adversarial_lists():
 
 
 def test_probe_search_is_a_lower_bound():
-    """The kernel's 32-probe boundary search finds the first task at or past the target, as a
-    binary search does: non-decreasing begins with runs of equal values (empty tasks), targets
+    """A 32-probe boundary search finds the first task at or past the target, as a binary search
+    does: non-decreasing begins with runs of equal values (empty tasks), targets
     before, between, on and past the begins."""
     rng = np.random.default_rng(5)
     for n in list(range(1, 70)) + [1000, 38281, 79199]:
